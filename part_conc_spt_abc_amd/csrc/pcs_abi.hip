@@ -77,23 +77,28 @@ int validate_proposal(const pcs_system& s, const pcs_proposal& p)
 }
 
 // Summed-area table of the observed histogram (uint32 like the reference's
-// host SAT, src/gpu/detail/simulation_impl.inl:617-628) and its deepest row.
-void build_sat(const uint32_t* H, uint32_t n_k, uint32_t n_de, std::vector<uint32_t>& S, uint32_t& maxrow)
+// host SAT, src/gpu/detail/simulation_impl.inl:617-628), in rows of
+// sat_pitch(n_de) with the columns at their right end, its deepest row and
+// its largest entry.
+void build_sat(const uint32_t* H, uint32_t n_k, uint32_t n_de, std::vector<uint32_t>& S, uint32_t& maxrow, uint32_t& most)
 {
-    S.assign((size_t)n_k * n_de, 0u);
-    maxrow = 0;
+    const uint32_t pitch = sat_pitch(n_de), pad = pitch - n_de;
+    S.assign((size_t)n_k * pitch, 0u);
+    maxrow = most = 0;
     for (uint32_t i = 0; i < n_k; ++i) {
         uint32_t run = 0;
+        uint32_t* row = S.data() + (size_t)i * pitch + pad;
         for (uint32_t j = 0; j < n_de; ++j) {
             const uint32_t h = H ? H[(size_t)i * n_de + j] : 0u;
             if (h) maxrow = i;
             run += h;
-            S[(size_t)i * n_de + j] = run + (i ? S[(size_t)(i - 1) * n_de + j] : 0u);
+            row[j] = run + (i ? row[(ptrdiff_t)j - (ptrdiff_t)pitch] : 0u);
+            most = std::max(most, row[j]);
         }
     }
 }
 
-DevSys make_devsys(const pcs_system& s, uint32_t maxrow, const uint32_t* dsat)
+DevSys make_devsys(const pcs_system& s, uint32_t maxrow, uint32_t most, const uint32_t* dsat)
 {
     DevSys d{};
     d.n_species = s.n_species;
@@ -111,6 +116,7 @@ DevSys make_devsys(const pcs_system& s, uint32_t maxrow, const uint32_t* dsat)
     d.dist_kind = s.dist_kind;
     d.maxrow_obs = maxrow;
     d.obs_sat = dsat;
+    d.obs_max = most;
     return d;
 }
 
@@ -206,6 +212,8 @@ struct pcs_batch {
     int last_mode = -1;
     bool ran = false;
     uint32_t reruns = 0;
+    // distance scratch: of the batch stream, then of each plain stream
+    DistScratch* d_dscratch = nullptr;
 };
 
 namespace {
@@ -342,7 +350,7 @@ int fetch_plan(pcs_batch* b)
     return PCS_OK;
 }
 
-DistArgs dist_args(pcs_batch* b, uint32_t lo, uint32_t n)
+DistArgs dist_args(pcs_batch* b, uint32_t lo, uint32_t n, int stream = 0)
 {
     DistArgs d{};
     d.sys = b->ctx->d_sys;
@@ -354,6 +362,7 @@ DistArgs dist_args(pcs_batch* b, uint32_t lo, uint32_t n)
     d.exact = b->d_exact;
     d.tracks = b->d_tracks;
     d.status = b->d_status;
+    d.scratch = b->d_dscratch + stream;
     return d;
 }
 
@@ -414,7 +423,7 @@ int enqueue_plain(pcs_batch* b, const std::vector<uint32_t>* subset, bool stream
         hipStream_t s = streams ? b->pstream[i % PCS_PLAIN_STREAMS] : b->stream;
         PCS_HIP(launch_walk(walk_args(b, lo, hi), (int)t.particles_per_lane, (int)t.waves_per_group, false, 0, gauss,
                             zref, s));
-        PCS_HIP(launch_distance(dist_args(b, P, 1), c->sys.n_k, c->sys.n_de, s));
+        PCS_HIP(launch_distance(dist_args(b, P, 1, streams ? 1 + (int)(i % PCS_PLAIN_STREAMS) : 0), c->sys.n_k, c->sys.n_de, s));
     }
     if (streams) {
         for (int k = 0; k < PCS_PLAIN_STREAMS; ++k) {
@@ -670,12 +679,12 @@ int pcs_open(const pcs_system* sys, const uint32_t* obs_hist, int device, pcs_ct
     hipDeviceGetAttribute(&c->n_cu, hipDeviceAttributeMultiprocessorCount, device);
     if (c->n_cu <= 0) c->n_cu = 256;
     std::vector<uint32_t> sat;
-    uint32_t maxrow = 0;
-    build_sat(obs_hist, sys->n_k, sys->n_de, sat, maxrow);
+    uint32_t maxrow = 0, most = 0;
+    build_sat(obs_hist, sys->n_k, sys->n_de, sat, maxrow, most);
     int r = dev_alloc(&c->d_sat, sat.size());
     if (r == PCS_OK) r = dev_alloc(&c->d_sys, 1);
     if (r == PCS_OK) {
-        c->dsys = make_devsys(*sys, maxrow, c->d_sat);
+        c->dsys = make_devsys(*sys, maxrow, most, c->d_sat);
         hipError_t e = hipMemcpy(c->d_sat, sat.data(), sat.size() * 4, hipMemcpyHostToDevice);
         if (e == hipSuccess) e = hipMemcpy(c->d_sys, &c->dsys, sizeof(DevSys), hipMemcpyHostToDevice);
         if (e == hipSuccess) e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
@@ -755,6 +764,11 @@ int pcs_batch_create(pcs_ctx* c, pcs_batch** out)
     int r = e == hipSuccess ? PCS_OK : hip_error(e, "pcs_batch_create");
     if (r == PCS_OK) r = dev_alloc(&b->d_seed, 1);
     if (r == PCS_OK) r = dev_alloc(&b->d_tile_counter, 1);
+    if (r == PCS_OK) r = dev_alloc(&b->d_dscratch, 1 + PCS_PLAIN_STREAMS);
+    if (r == PCS_OK) {
+        e = hipMemset(b->d_dscratch, 0, (1 + PCS_PLAIN_STREAMS) * sizeof(DistScratch));
+        if (e != hipSuccess) r = hip_error(e, "pcs_batch_create");
+    }
     if (r != PCS_OK) {
         pcs_batch_destroy(b);
         return r;
@@ -775,7 +789,7 @@ int pcs_batch_destroy(pcs_batch* b)
     void* ptrs[] = {b->d_props, b->d_vframes, b->d_vparticles, b->d_vprop, b->d_vtile, b->d_rec, b->d_srt,
                     b->d_rec2, b->d_srt2, b->d_count, b->d_tracks, b->d_tile_counter, b->d_dist, b->d_exact, b->d_status,
                     b->d_seed, b->d_in, b->d_theta_pop, b->d_cumw, b->d_theta_new, b->d_totals, b->d_wpop,
-                    b->d_xn, b->d_xo, b->d_wsum, b->d_part};
+                    b->d_xn, b->d_xo, b->d_wsum, b->d_part, b->d_dscratch};
     for (void* p : ptrs)
         if (p) hipFree(p);
     if (b->h_seed) hipHostFree(b->h_seed);

@@ -11,6 +11,14 @@ namespace pcs {
 
 constexpr int kWave = 64;
 
+// A wave's row sweep (distance_split) gives each of its 64 lanes dist_cpl(n_de)
+// columns, for histograms of up to 1,024. Rows of the observed table are then
+// 64 dist_cpl(n_de) long, the n_de columns at their right end and zeros before
+// them: a column left of the first bin holds 0 in both tables and adds nothing,
+// so no lane is masked and rows are read 16 bytes at a time.
+__host__ __device__ inline uint32_t dist_cpl(uint32_t n_de) { return n_de <= 256u ? 4u : (n_de <= 512u ? 8u : 16u); }
+__host__ __device__ inline uint32_t sat_pitch(uint32_t n_de) { return n_de <= 1024u ? 64u * dist_cpl(n_de) : n_de; }
+
 // One model, resident in HBM (one entry per system of a context or server).
 struct DevSys {
     uint32_t n_species, kmin, n_k, n_de;
@@ -21,8 +29,9 @@ struct DevSys {
     float detect_sigma;
     uint32_t dist_kind;
     uint32_t maxrow_obs;      // last row holding observed tracks (0 if none)
-    const uint32_t* obs_sat;  // observed summed-area table, n_k * n_de uint32
-    uint64_t pad1;
+    const uint32_t* obs_sat;  // observed summed-area table, n_k rows of sat_pitch(n_de) uint32
+    uint32_t obs_max;         // its largest entry
+    uint32_t pad1;
 };
 static_assert(sizeof(DevSys) == 80, "DevSys layout");
 
@@ -98,6 +107,16 @@ struct WalkArgs {
     const uint64_t* tile_total; // persistent form, nullable: tiles planned on the device (caps tile_hi)
 };
 
+// Partial sums of simulations that several distance workgroups share: slot
+// 2 (job parts + part) holds a part's sum (low, high); ticket[job] counts the
+// parts done, zero between launches (the last part sets it back). For the
+// launches of one stream, which run one after the other.
+constexpr uint32_t kDistSlots = 1024, kDistMaxParts = 16;
+struct DistScratch {
+    uint64_t sum[2 * kDistSlots];
+    uint32_t ticket[kDistSlots];
+};
+
 struct DistArgs {
     const DevSys* sys;
     const DevProp* props;
@@ -108,9 +127,14 @@ struct DistArgs {
     uint64_t* exact;            // integer sum per proposal
     uint32_t* tracks;           // binned tracks per proposal
     int32_t* status;            // PCS_OK or PCS_EOVERFLOW per proposal
-    uint32_t colh_off;          // LDS word offset of the column histogram (set by launch_distance)
-    uint32_t srtl_off;          // LDS word offset of the sorted bins (set by launch_distance)
-    uint32_t srtl_cap;          // sorted 16-bit bins that fit in LDS (set by launch_distance)
+    DistScratch* scratch;       // nullable: then one workgroup per simulation
+    // set by launch_distance: workgroups per simulation, LDS word offsets (see
+    // DistLds, SplitLds), sorted 16-bit bins that fit in LDS
+    uint32_t parts;
+    uint32_t colh_off;
+    uint32_t piece_off, diff_off, base_off, misc_off;
+    uint32_t srtl_off;
+    uint32_t srtl_cap;
 };
 
 // ------------------------------------------------ device-resident request loop

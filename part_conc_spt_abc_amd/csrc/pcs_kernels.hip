@@ -35,6 +35,7 @@
 #include <algorithm>
 #include <map>
 #include <mutex>
+#include <tuple>
 #include <type_traits>
 #include <utility>
 
@@ -849,6 +850,49 @@ __global__ __launch_bounds__(256) void walk_kernel(WalkArgs a)
     }
 }
 
+// Loads and stores at agent (device) and system scope, for data that other
+// workgroups or the host read and write meanwhile.
+__device__ __forceinline__ uint64_t bcast64(uint64_t v)
+{
+    return ((uint64_t)uniform((uint32_t)(v >> 32)) << 32) | (uint64_t)uniform((uint32_t)v);
+}
+
+__device__ __forceinline__ uint64_t ld_agent64(const uint64_t* p)
+{
+    return __hip_atomic_load(const_cast<uint64_t*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__device__ __forceinline__ uint32_t ld_agent32(const uint32_t* p)
+{
+    return __hip_atomic_load(const_cast<uint32_t*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__device__ __forceinline__ uint64_t ld_system64(const uint64_t* p)
+{
+    return __hip_atomic_load(const_cast<uint64_t*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+__device__ __forceinline__ uint32_t ld_system32(const uint32_t* p)
+{
+    return __hip_atomic_load(const_cast<uint32_t*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+__device__ __forceinline__ void st_agent32(uint32_t* p, uint32_t v)
+{
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__device__ __forceinline__ void st_agent64(uint64_t* p, uint64_t v)
+{
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__device__ __forceinline__ bool cas_agent64(uint64_t* p, uint64_t expect, uint64_t want)
+{
+    return __hip_atomic_compare_exchange_strong(p, &expect, want, __ATOMIC_ACQ_REL, __ATOMIC_RELAXED,
+                                                __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // --------------------------------------------------------------- distance
 
 constexpr int kDistThreads = 256;
@@ -875,6 +919,7 @@ __device__ __forceinline__ uint32_t wave_incl_scan(uint32_t v)
     return (uint32_t)x;
 }
 
+template <int NW = kDistThreads / kWave>
 __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t* wsum, uint32_t& total)
 {
     const uint32_t lane = threadIdx.x % kWave, wave = threadIdx.x / kWave;
@@ -883,7 +928,7 @@ __device__ __forceinline__ uint32_t block_excl_scan(uint32_t v, uint32_t* wsum, 
     __syncthreads();
     uint32_t base = 0u, tot = 0u;
 #pragma unroll
-    for (int w = 0; w < kDistThreads / kWave; ++w) {
+    for (int w = 0; w < NW; ++w) {
         const uint32_t s = wsum[w];
         base += ((uint32_t)w < wave) ? s : 0u;
         tot += s;
@@ -1064,7 +1109,8 @@ __device__ __forceinline__ DistOut distance_block(const DevProp& pr, const DevSy
     const uint32_t j0 = tid * SEG;
     uint64_t acc = 0ull, acc_hi = 0ull;
     const bool l1 = sy.dist_kind == PCS_DIST_L1;
-    const auto* R = gview(sy.obs_sat);
+    const uint32_t pitch = sat_pitch(n_de);
+    const auto* R = gview(sy.obs_sat) + (pitch - n_de);
     const uint32_t maxrow_obs = sy.maxrow_obs;
     const uint32_t lane = tid % kWave;
 #if PCS_TRACE
@@ -1096,7 +1142,7 @@ __device__ __forceinline__ DistOut distance_block(const DevProp& pr, const DevSy
         constexpr int PF = 2;
         uint32_t rb[PF][SEG];
         auto load_row = [&](uint32_t (&dst)[SEG], uint32_t row) {
-            const auto* Rrow = R + (uint64_t)row * n_de;
+            const auto* Rrow = R + (uint64_t)row * pitch;
 #pragma unroll
             for (int m = 0; m < SEG; ++m) dst[m] = Rrow[min(j0 + (uint32_t)m, n_de - 1u)];
         };
@@ -1328,6 +1374,580 @@ void distance_kernel(DistArgs a)
     }
 }
 
+// ------------------------------------------- distance of few simulations
+
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4u __attribute__((ext_vector_type(4), aligned(4)));  // a quad at any record
+
+// Rows with at most this many records enter a lane's columns by comparison,
+// others through the wave's column histogram in LDS.
+constexpr uint32_t kSplitSparseRow = 3;
+
+// Row counters of the first rows, where most records are (short tracks), come
+// four to a row, lane l using number l % 4: 64 records of a wave hit few
+// distinct rows, and LDS atomics on one word run one after the other. (One
+// counter a row: the counting pass over 104,000 records of a lone simulation
+// took 24 us, the scatter 31 us.)
+constexpr uint32_t kSubRows = 256, kSub = 4;
+__host__ __device__ inline uint32_t row_counters(uint32_t n_k) { return n_k + (n_k < kSubRows ? n_k : kSubRows) * (kSub - 1u); }
+__device__ __forceinline__ uint32_t row_counter(uint32_t r) { return r + min(r, kSubRows) * (kSub - 1u); }  // row r's first
+
+// LDS words of the counters, and of the counters and the rows' waves.
+__host__ __device__ inline uint32_t counter_words(uint32_t n_k) { return (row_counters(n_k) + 3u) & ~3u; }
+__host__ __device__ inline uint32_t rows_words(uint32_t n_k) { return counter_words(n_k) + (((n_k + 15u) / 16u) << 2); }
+
+// LDS working set of the distance of one simulation, for a workgroup of NW
+// waves: row counters / row offsets (row_counters(n_k)), the wave that sweeps
+// each row (n_k bytes), a column histogram of 64 * CPL words per wave, the
+// column counts of the rows before this workgroup's (a row pitch; only when
+// several workgroups share a simulation), kSplitMisc words - per-wave scan
+// partials (kSplitWaves), the deepest occupied row and, from word 32 on, the
+// final reduction - and room for the bins sorted by row (srtl_cap 16-bit
+// entries; more are sorted into the slice's HBM scratch instead).
+struct SplitLds {
+    uint32_t* rowc;
+    uint8_t* piece;
+    uint32_t* diff;
+    uint32_t* base;
+    uint32_t* misc;
+    uint16_t* srtl;
+    uint32_t srtl_cap;
+};
+constexpr int kSplitWaves = 16;
+constexpr int kSplitMisc = 32 + 4 * kSplitWaves;
+
+// A lane's CPL columns in LDS (16-byte aligned).
+template <int CPL>
+__device__ __forceinline__ void load_cols(uint32_t (&c)[CPL], const uint32_t* p)
+{
+#pragma unroll
+    for (int q = 0; q < CPL / 4; ++q) {
+        const u32x4 x = reinterpret_cast<const u32x4*>(p)[q];
+#pragma unroll
+        for (int m = 0; m < 4; ++m) c[4 * q + m] = x[m];
+    }
+}
+template <int CPL>
+__device__ __forceinline__ void zero_cols(uint32_t* p)
+{
+#pragma unroll
+    for (int q = 0; q < CPL / 4; ++q) reinterpret_cast<u32x4*>(p)[q] = u32x4{0u, 0u, 0u, 0u};
+}
+
+// Exact distance of one simulation's record slice against the observed
+// summed-area table, by a workgroup of NW waves, or its part of it where
+// `parts` workgroups share the simulation. CPL = dist_cpl(n_de).
+//
+// The rows are what is split: each wave of the simulation's workgroups takes a
+// contiguous piece of them, of about the same cost, which it sweeps alone -
+// 64 lanes x CPL columns, the running column sums of the cumulative histogram
+// in registers, no barrier from row to row. (The block form sweeps row after
+// row with a barrier or two each: 3 simulations of 104,000 records at H
+// 1000x1000 took 400 us, now 88.) What bounds it now are the two passes over
+// the records: LDS atomics, 8 to 12 cycles for a wave's 64. A wave's starting column sums are the
+// column histogram of the records before its first row: of the rows before the
+// workgroup's (counted by the scatter; none for part 0), plus the earlier
+// waves' histograms of their own records (counted by the scatter too).
+//
+// The slice is read from HBM once when it holds at most KREG records a thread
+// (held in registers between the row count and the scatter); records past that
+// are read a second time. Both reads take four records a load: a slice is read
+// by few waves, so what they keep in flight is what sets its pace. The scatter
+// writes the 16-bit bins of the workgroup's rows sorted by row into LDS when
+// they fit L.srtl_cap, else into the slice's HBM scratch at the place the whole
+// slice's order gives them. Within a row the order of the bins depends on the
+// atomics; the sum depends only on counts.
+template <int CPL, int NW, int KREG>
+__device__ __forceinline__ DistOut distance_split(const DevProp& pr, const DevSys& sy, uint32_t count, const SplitLds& L,
+                                                  uint32_t part, uint32_t parts)
+{
+    constexpr uint32_t kThreads = (uint32_t)NW * kWave;
+    constexpr uint32_t W = 64u * CPL;
+    uint32_t* rowc = L.rowc;
+    uint32_t* wsum = L.misc;
+    uint32_t* smax = L.misc + kSplitWaves;
+    uint64_t* red = reinterpret_cast<uint64_t*>(L.misc + 32);
+    const uint32_t tid = threadIdx.x, lane = tid % kWave, wave = uniform(tid / kWave);
+    const uint32_t n_k = sy.n_k, n_de = sy.n_de, mo = sy.maxrow_obs;
+    const uint32_t pitch = sat_pitch(n_de), pad = pitch - n_de;  // columns are right-aligned in the pitch
+    const auto* rec = gview(pr.rec);
+    uint32_t* D = L.diff + wave * W;
+
+    if (count > pr.rec_cap)  // record slice overflowed: counted, not stored
+        return DistOut{0ull, 0ull, count, PCS_EOVERFLOW};
+    const uint32_t T = count;
+    // Issue priority over walking waves that share the SIMDs: a distance is
+    // one workgroup on the critical path of its simulation's latency.
+    __builtin_amdgcn_s_setprio(3);
+
+    const uint32_t n_c = row_counters(n_k);
+    for (uint32_t i = tid; i < n_c; i += kThreads) rowc[i] = 0u;
+    for (uint32_t i = tid; i < (uint32_t)NW * W; i += kThreads) L.diff[i] = 0u;
+    if (parts > 1u)
+        for (uint32_t i = tid; i < pitch; i += kThreads) L.base[i] = 0u;
+    if (tid == 0) *smax = 0u;
+    __syncthreads();
+
+    // Row counts and the deepest occupied row. Thread t takes quads t, t +
+    // kThreads, ... of the slice. A quad's load is issued for every slot, at an
+    // index clamped into the slice, and masked afterwards: a load under a lane
+    // mask would be waited for before the next one is issued. The last quad is
+    // moved back to end with the slice; the records it shares with the one
+    // before, and the slots past the slice, read as kNoRecord (row 0xffff >
+    // PCS_MAX_NK). A slice of under four records is read a record a quad.
+    constexpr uint32_t kNoRecord = ~0u;
+    const uint32_t nq = (T + 3u) / 4u;
+    auto load_quad = [&](uint32_t q, uint32_t (&v)[4]) {
+        if (T >= 4u) {
+            const uint32_t at = min(4u * q, T - 4u);
+            const u32x4u x = *(const __attribute__((address_space(1))) u32x4u*)(rec + at);
+#pragma unroll
+            for (uint32_t j = 0; j < 4u; ++j) v[j] = (q < nq && at + j >= 4u * q) ? x[j] : kNoRecord;
+        } else {
+#pragma unroll
+            for (uint32_t j = 0; j < 4u; ++j) v[j] = 4u * q + j < T ? rec[4u * q + j] : kNoRecord;
+        }
+    };
+    // The scatter takes the held words through an empty asm statement, so
+    // that nothing the count derived from them (rows, lane masks) is kept
+    // alive across the scan in place of being recomputed.
+    constexpr uint32_t HQ = KREG / 4;  // quads held a thread
+    uint32_t held[HQ > 0u ? HQ : 1u][4];
+    uint32_t mr = 0u;
+    const uint32_t sub = lane % kSub;
+    auto counter = [&](uint32_t r) -> uint32_t { return row_counter(r) + (r < kSubRows ? sub : 0u); };
+    auto tally = [&](uint32_t v) {
+        if (v == kNoRecord) return;
+        const uint32_t r = v >> 16;
+        atomicAdd(&rowc[counter(r)], 1u);
+        mr = max(mr, r);
+    };
+#pragma unroll
+    for (uint32_t u = 0; u < HQ; ++u) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) held[u][j] = kNoRecord;
+        if (u * kThreads < nq) load_quad(u * kThreads + tid, held[u]);
+    }
+#pragma unroll
+    for (uint32_t u = 0; u < HQ; ++u)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) tally(held[u][j]);
+    // Past the held quads: kLoads a thread at a time, the next ones on their
+    // way while these are counted.
+    constexpr uint32_t kLoads = 3u;
+    auto rest = [&](auto&& take) {
+        uint32_t v[kLoads][4];
+#pragma unroll
+        for (uint32_t u = 0; u < kLoads; ++u) load_quad(HQ * kThreads + u * kThreads + tid, v[u]);
+        for (uint32_t q0 = HQ * kThreads; q0 < nq; q0 += kLoads * kThreads) {
+            uint32_t n[kLoads][4];
+#pragma unroll
+            for (uint32_t u = 0; u < kLoads; ++u) load_quad(q0 + (kLoads + u) * kThreads + tid, n[u]);
+#pragma unroll
+            for (uint32_t u = 0; u < kLoads; ++u)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    take(v[u][j]);
+                    v[u][j] = n[u][j];
+                }
+        }
+    };
+    if (HQ * kThreads < nq) rest(tally);
+#pragma unroll
+    for (int o = kWave / 2; o > 0; o >>= 1) mr = max(mr, (uint32_t)__shfl_xor((int)mr, o, kWave));
+    if (lane == 0u) atomicMax(smax, mr);
+    __syncthreads();
+
+    // Exclusive scan of the counters, which become the first slots of their
+    // records in the order by rows.
+    {
+        const uint32_t ch = (n_c + kThreads - 1) / kThreads;
+        const uint32_t b0 = min(tid * ch, n_c), b1 = min(b0 + ch, n_c);
+        uint32_t run = 0u;
+        for (uint32_t i = b0; i < b1; ++i) run += rowc[i];
+        uint32_t tot;
+        uint32_t ex = block_excl_scan<NW>(run, wsum, tot);
+        for (uint32_t i = b0; i < b1; ++i) {
+            const uint32_t c = rowc[i];
+            rowc[i] = ex;
+            ex += c;
+        }
+    }
+    __syncthreads();
+
+    // Rows [0, r_end) hold records or differ in the observed table; the rows
+    // after them, up to n_k, repeat the last. They are split over all the
+    // simulation's waves by cost: 8 a row that is summed (every row up to the
+    // deepest observed one; past it each record's, at most), 1 per 16 records.
+    const uint32_t deep = uniform(*smax);
+    const uint32_t r_end = max(deep, mo) + 1u;  // <= n_k
+    const uint32_t mo1 = mo + 1u;               // end of the rows that are all summed
+    auto first_slot = [&](uint32_t r) -> uint32_t { return r < n_k ? rowc[row_counter(r)] : T; };  // records before row r
+    const uint32_t obs_rec = uniform(first_slot(mo1));
+    constexpr uint32_t kRowCost = 8u;
+    auto cost = [&](uint32_t r) -> uint32_t {
+        const uint32_t n = first_slot(r);
+        return kRowCost * (min(r, mo1) + (r > mo1 ? min(r - mo1, n - obs_rec) : 0u)) + n / 16u;
+    };
+    const uint64_t tot = cost(r_end);
+    // first row whose cost before it reaches piece k's share
+    auto piece = [&](uint32_t k) -> uint32_t {
+        const uint64_t t = tot * k / (parts * (uint32_t)NW);
+        if (k == 0u) return 0u;
+        for (uint32_t b = 0u; b < r_end; b += (uint32_t)kWave) {
+            const uint32_t r = min(b + lane, r_end);
+            const uint64_t m = ballot((uint64_t)cost(r) >= t);
+            if (m != 0ull) return min(b + (uint32_t)__builtin_ctzll(m), r_end);
+        }
+        return r_end;
+    };
+    const uint32_t k0 = part * (uint32_t)NW;
+    const uint32_t r_lo = uniform(parts > 1u ? piece(k0) : 0u);                              // the workgroup's rows
+    const uint32_t r_hi = uniform(part + 1u < parts ? piece(k0 + (uint32_t)NW) : n_k);
+    const uint32_t ra = uniform(piece(k0 + wave)), rz = uniform(wave + 1u < (uint32_t)NW ? piece(k0 + wave + 1u) : min(r_hi, r_end));
+    const uint32_t nlow = uniform(first_slot(r_lo)), town = uniform(first_slot(r_hi)) - nlow;
+    const uint32_t stop = wave + 1u == (uint32_t)NW ? r_hi : rz;  // the very last wave's rows go on to n_k
+    for (uint32_t r = ra + lane; r < rz; r += (uint32_t)kWave) L.piece[r] = (uint8_t)wave;
+    __syncthreads();  // before the scatter moves the offsets
+
+    // Scatter bins by row; afterwards the last counter of row r of the
+    // workgroup's rows is one past the row's last slot. Each record also goes
+    // into the column counts of its row's wave, those of earlier rows into the
+    // workgroup's starting counts.
+    const bool in_lds = town <= L.srtl_cap;
+    uint16_t* srtl = L.srtl;
+    auto* srtg = gview(reinterpret_cast<uint16_t*>(pr.srt)) + nlow;
+    auto put = [&](uint32_t v) {
+        if (v == kNoRecord) return;
+        const uint32_t r = v >> 16;
+        if (r >= r_lo && r < r_hi) {
+            const uint32_t pos = atomicAdd(&rowc[counter(r)], 1u) - nlow;
+            if (in_lds) srtl[pos] = (uint16_t)v;
+            else srtg[pos] = (uint16_t)v;
+            atomicAdd(&L.diff[L.piece[r] * W + pad + (v & 0xffffu)], 1u);
+        } else if (r < r_lo) {
+            atomicAdd(&L.base[pad + (v & 0xffffu)], 1u);
+        }
+    };
+#pragma unroll
+    for (uint32_t u = 0; u < HQ; ++u)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            uint32_t v = held[u][j];
+            asm volatile("" : "+v"(v));
+            put(v);
+        }
+    if (HQ * kThreads < nq) rest(put);
+    __threadfence_block();
+    __syncthreads();
+#if PCS_TRACE
+    const uint64_t t_sweep = wall_clock64();
+#endif
+
+    uint64_t acc = 0ull, acc_hi = 0ull;
+    const bool l1 = sy.dist_kind == PCS_DIST_L1;
+    const auto* R = gview(sy.obs_sat);
+    // Cumulative counts stay below 2^20 nearly always; a lane's sum over all
+    // rows (CPL x 4,096 x 2^40 at most) then fits 64 bits. Above, 128 bits.
+    const bool wide = max(T, sy.obs_max) >= (1u << 20);
+    auto bin_at = [&](uint32_t t) -> uint32_t {
+        if (in_lds) return (uint32_t)srtl[t];
+        return (uint32_t)srtg[t];
+    };
+
+    // The column counts of the records before the wave's rows, then (the
+    // scatter's counts taken) its own histogram zero again.
+    uint32_t Ccol[CPL];
+#pragma unroll
+    for (int m = 0; m < CPL; ++m) Ccol[m] = 0u;
+    if (parts > 1u) load_cols<CPL>(Ccol, L.base + lane * CPL);
+    for (uint32_t v = 0; v < wave; ++v) {
+        uint32_t c[CPL];
+        load_cols<CPL>(c, L.diff + v * W + lane * CPL);
+#pragma unroll
+        for (int m = 0; m < CPL; ++m) Ccol[m] += c[m];
+    }
+    __syncthreads();
+    zero_cols<CPL>(D + lane * CPL);
+    wave_lds_sync();
+    // running sums of the lane's columns, then over the lanes before it
+    auto prefix = [&](uint32_t (&c)[CPL]) -> uint32_t {
+#pragma unroll
+        for (int m = 1; m < CPL; ++m) c[m] += c[m - 1];
+        return wave_incl_scan(c[CPL - 1]) - c[CPL - 1];
+    };
+    {
+        const uint32_t ex = prefix(Ccol);
+#pragma unroll
+        for (int m = 0; m < CPL; ++m) Ccol[m] += ex;
+    }
+
+    auto load_row = [&](uint32_t (&dst)[CPL], uint32_t row) {
+        const auto* p = (const __attribute__((address_space(1))) u32x4*)(R + (uint64_t)row * pitch + lane * CPL);
+#pragma unroll
+        for (int q = 0; q < CPL / 4; ++q) {
+            const u32x4 x = p[q];
+#pragma unroll
+            for (int m = 0; m < 4; ++m) dst[4 * q + m] = x[m];
+        }
+    };
+    // Column pairs (j0 + 2p, j0 + 2p + 1) as 16-bit halves (columns and
+    // per-row counts stay below 2^15): jp holds j0 + 1 and j0 + 2, and
+    // pair p compares them with the bin less 2p.
+    constexpr int NP = CPL / 2;
+    const uint32_t j0 = lane * CPL;
+    const u16x2 jp{(uint16_t)(j0 + 1u), (uint16_t)(j0 + 2u)};
+    // Records of slots [s0, s1), the lane's own slot of them (clamped)
+    // given, into the column sums.
+    auto add_bins = [&](uint32_t s0, uint32_t s1, uint32_t mine) {
+        const uint32_t nr = s1 - s0;
+        if (nr <= kSplitSparseRow) {
+            // bin - (column + 1) is negative, the half's top bit, exactly
+            // when the bin is at or left of the column (it lies in
+            // (-2^12, 2^12) as a 16-bit difference)
+            u16x2 h[NP];
+#pragma unroll
+            for (int p = 0; p < NP; ++p) h[p] = u16x2{0, 0};
+            for (uint32_t q = 0u; q < nr; ++q) {
+                const uint32_t b = (uint32_t)__builtin_amdgcn_readlane((int)mine, (int)q) + pad;
+#pragma unroll
+                for (int p = 0; p < NP; ++p) {
+                    const uint16_t bp = (uint16_t)(b - 2u * (uint32_t)p);
+                    h[p] += (u16x2)(u16x2{bp, bp} - jp) >> (uint16_t)15;
+                }
+            }
+#pragma unroll
+            for (int m = 0; m < CPL; ++m) Ccol[m] += (m & 1) ? (uint32_t)h[m / 2].y : (uint32_t)h[m / 2].x;
+            return;
+        }
+        if (lane < nr) atomicAdd(&D[mine + pad], 1u);
+        // past the first 64, 8 bins a lane in flight, as HBM-resident ones need
+        for (uint32_t t0 = s0 + (uint32_t)kWave; t0 < s1; t0 += 8u * kWave) {
+            uint32_t b[8];
+            if (in_lds) {
+#pragma unroll
+                for (int u = 0; u < 8; ++u) b[u] = srtl[min(t0 + lane + (uint32_t)(u * kWave), s1 - 1u)];
+            } else {
+#pragma unroll
+                for (int u = 0; u < 8; ++u) b[u] = srtg[min(t0 + lane + (uint32_t)(u * kWave), s1 - 1u)];
+            }
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                if (t0 + lane + (uint32_t)(u * kWave) < s1) atomicAdd(&D[b[u] + pad], 1u);
+        }
+        wave_lds_sync();
+        uint32_t v[CPL];
+        load_cols<CPL>(v, D + lane * CPL);
+        wave_lds_sync();
+        zero_cols<CPL>(D + lane * CPL);
+        wave_lds_sync();
+        const uint32_t ex = prefix(v);
+#pragma unroll
+        for (int m = 0; m < CPL; ++m) Ccol[m] += ex + v[m];
+    };
+    struct RowSum {
+        uint64_t lo, hi;
+    };
+    auto row_sum = [&](const uint32_t (&rv)[CPL]) -> RowSum {
+        uint64_t s = 0ull, s_hi = 0ull;
+        if (!wide) {
+            if (l1) {
+                uint32_t t = 0u;
+#pragma unroll
+                for (int m = 0; m < CPL; ++m) t += max(Ccol[m], rv[m]) - min(Ccol[m], rv[m]);
+                s = t;
+            } else {
+                int64_t t = 0;
+#pragma unroll
+                for (int m = 0; m < CPL; ++m) {
+                    const int32_t dd = (int32_t)(Ccol[m] - rv[m]);
+                    t += (int64_t)dd * dd;
+                }
+                s = (uint64_t)t;
+            }
+        } else {
+#pragma unroll
+            for (int m = 0; m < CPL; ++m) {
+                const uint32_t dd = max(Ccol[m], rv[m]) - min(Ccol[m], rv[m]);
+                add128(s, s_hi, l1 ? (uint64_t)dd : (uint64_t)dd * dd, 0ull);
+            }
+        }
+        return RowSum{s, s_hi};
+    };
+    // A row's sum counted for w rows: acc += w r (wide: in three 32 x 32 ->
+    // 64-bit multiply-adds; r.hi < CPL, as a row sums CPL squares below 2^64).
+    auto add_rows = [&](const RowSum& r, uint32_t w) {
+        if (!wide) {
+            acc += r.lo * w;
+            return;
+        }
+        const uint64_t p0 = (uint64_t)(uint32_t)r.lo * w;
+        const uint64_t p1 = (uint64_t)(uint32_t)(r.lo >> 32) * w + (p0 >> 32);
+        const uint64_t ph = (uint64_t)(uint32_t)r.hi * w + (p1 >> 32);
+        add128(acc, acc_hi, (p1 << 32) | (uint32_t)p0, ph);
+    };
+    // Row slots, 64 rows at a time: lane l holds the first slot and the end
+    // of row gb + l.
+    uint32_t gb = ra - (uint32_t)kWave, gs = 0u, ge = 0u;
+    auto group = [&](uint32_t b) {
+        gb = b;
+        const uint32_t r = min(b + lane, n_k - 1u);
+        ge = rowc[row_counter(r + 1u) - 1u] - nlow;
+        gs = r > r_lo ? rowc[row_counter(r) - 1u] - nlow : 0u;
+    };
+    struct Row {
+        uint32_t i, s0, s1, bin;
+    };
+    auto fetch = [&](uint32_t i) -> Row {
+        const uint32_t l = i - gb;
+        const uint32_t s0 = (uint32_t)__builtin_amdgcn_readlane((int)gs, (int)l);
+        const uint32_t s1 = (uint32_t)__builtin_amdgcn_readlane((int)ge, (int)l);
+        uint32_t b = 0u;
+        if (s1 != s0) b = bin_at(min(s0 + lane, town - 1u));
+        return Row{i, s0, s1, b};
+    };
+
+    // Rows up to the deepest observed one: each is summed. Observed rows
+    // are loaded two ahead into a ring of registers, the next row's slots
+    // and first bins one ahead.
+    const uint32_t ez = min(rz, mo1);
+    constexpr uint32_t PF = 2u;
+    uint32_t rb[PF][CPL];
+    if (ra < ez) {
+#pragma unroll
+        for (uint32_t d = 0; d < PF; ++d) load_row(rb[d], min(ra + d, mo));
+        group(ra);
+        Row next = fetch(ra);
+        for (uint32_t i0 = ra; i0 < ez; i0 += PF) {
+#pragma unroll
+            for (uint32_t d = 0; d < PF; ++d) {
+                const uint32_t i = i0 + d;
+                if (i >= ez) break;
+                const Row cur = next;
+                if (i + 1u < ez) {
+                    if (i + 1u - gb >= (uint32_t)kWave) group(i + 1u);
+                    next = fetch(i + 1u);
+                }
+                if (cur.s1 != cur.s0) add_bins(cur.s0, cur.s1, cur.bin);
+                const RowSum rs = row_sum(rb[d]);
+                if (!wide) acc += rs.lo;
+                else add128(acc, acc_hi, rs.lo, rs.hi);
+                if (i + PF < ez) load_row(rb[d], i + PF);
+            }
+        }
+    }
+    // Rows past it: the observed table repeats row mo, so a row without
+    // records adds what the row above it did. The rows with records are
+    // found 64 at a time by one ballot, each one's bins read while the one
+    // before it is summed; a state of the columns is counted for all its rows.
+    uint32_t p = max(ra, mo1);
+    if (p < stop) {
+        load_row(rb[0], mo);
+        RowSum rs = row_sum(rb[0]);
+        const uint32_t z = min(rz, deep + 1u);
+        uint64_t mask = 0ull;
+        gb = p - (uint32_t)kWave;
+        auto next_row = [&]() -> Row {
+            while (mask == 0ull && gb + (uint32_t)kWave < z) {
+                group(gb + (uint32_t)kWave);
+                mask = ballot(gb + lane < z && ge != gs);
+            }
+            if (mask == 0ull) return Row{~0u, 0u, 0u, 0u};
+            const uint32_t l = (uint32_t)__builtin_ctzll(mask);
+            mask &= mask - 1ull;
+            return fetch(gb + l);
+        };
+        Row next = next_row();
+        while (next.i != ~0u) {
+            const Row cur = next;
+            next = next_row();
+            add_rows(rs, cur.i - p);
+            p = cur.i;
+            add_bins(cur.s0, cur.s1, cur.bin);
+            rs = row_sum(rb[0]);
+        }
+        add_rows(rs, stop - p);
+    }
+
+    // 128-bit sum over the block: across each wave by shuffles, then the
+    // waves' partial sums in LDS.
+#pragma unroll
+    for (int o = kWave / 2; o > 0; o >>= 1) {
+        const uint64_t l2 = __shfl_xor(acc, o, kWave), h2 = __shfl_xor(acc_hi, o, kWave);
+        add128(acc, acc_hi, l2, h2);
+    }
+    if (lane == 0u) {
+        red[wave] = acc;
+        red[kSplitWaves + wave] = acc_hi;
+    }
+    __syncthreads();
+    uint64_t lo = 0ull, hi = 0ull;
+    for (uint32_t w = 0; w < (uint32_t)NW; ++w) add128(lo, hi, red[w], red[kSplitWaves + w]);
+    __syncthreads();
+    __builtin_amdgcn_s_setprio(0);
+    DistOut o{lo, hi, T, PCS_OK};
+#if PCS_TRACE
+    o.t_sweep = t_sweep;
+#endif
+    return o;
+}
+
+// The distance at the model's own column width, in a kernel whose models have
+// at most 64 * CPL columns a pass.
+template <int CPL, int NW, int KREG>
+__device__ __forceinline__ DistOut split_any(const DevProp& pr, const DevSys& sy, uint32_t count, const SplitLds& L,
+                                             uint32_t part, uint32_t parts)
+{
+    if constexpr (CPL > 4) {
+        if (dist_cpl(sy.n_de) < (uint32_t)CPL)
+            return split_any<CPL / 2, NW, KREG>(pr, sy, count, L, part, parts);
+    }
+    return distance_split<CPL, NW, KREG>(pr, sy, count, L, part, parts);
+}
+
+// `a.parts` workgroups of NW waves per simulation (neighbouring blocks), whose
+// sums the last to finish adds up. Dynamic LDS as laid out by SplitLds, sized
+// to the models of the launch.
+template <int CPL, int NW>
+__global__ __launch_bounds__(NW * kWave) void distance_split_kernel(DistArgs a)
+{
+    extern __shared__ __align__(16) uint32_t split_lds[];
+    uint32_t* w = split_lds;
+    const SplitLds L{w,
+                     reinterpret_cast<uint8_t*>(w + a.piece_off),
+                     w + a.diff_off,
+                     w + a.base_off,
+                     w + a.misc_off,
+                     reinterpret_cast<uint16_t*>(w + a.srtl_off),
+                     a.srtl_cap};
+    const uint32_t job = blockIdx.x / a.parts, part = blockIdx.x % a.parts;
+    const uint32_t P = a.prop_lo + job;
+    const DevProp& pr = a.props[P];
+    DistOut o = split_any<CPL, NW, 8>(pr, a.sys[pr.sys_id], a.rec_count[P], L, part, a.parts);
+    if (threadIdx.x != 0) return;
+    if (a.parts > 1u) {
+        if (o.status == PCS_OK) {
+            uint64_t* slot = a.scratch->sum + 2u * (uint64_t)blockIdx.x;
+            st_agent64(slot, o.lo);
+            st_agent64(slot + 1, o.hi);
+            const uint32_t t = __hip_atomic_fetch_add(&a.scratch->ticket[job], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+            if (t + 1u != a.parts) return;
+            st_agent32(&a.scratch->ticket[job], 0u);  // as the next launch expects it
+            o.lo = o.hi = 0ull;
+            for (uint32_t q = 0; q < a.parts; ++q) {
+                const uint64_t* s = a.scratch->sum + 2u * ((uint64_t)job * a.parts + q);
+                add128(o.lo, o.hi, ld_agent64(s), ld_agent64(s + 1));
+            }
+        } else if (part != 0u) {
+            return;
+        }
+    }
+    a.exact[P] = dist_exact(o);  // an overflowed slice is rerun by the host
+    a.dist[P] = dist_log10(o);
+    a.tracks[P] = o.tracks;
+    a.status[P] = o.status;
+}
+
 // ------------------------------------------------------------ request loop
 //
 // serve_loop_kernel is the device-resident form of the serving loop: a
@@ -1342,47 +1962,6 @@ void distance_kernel(DistArgs a)
 // worker after idle_ticks in which no group claimed a tile).
 
 enum : uint32_t { kLoopIdle = 0u, kLoopWork = 1u, kLoopExit = 2u };
-
-__device__ __forceinline__ uint64_t bcast64(uint64_t v)
-{
-    return ((uint64_t)uniform((uint32_t)(v >> 32)) << 32) | (uint64_t)uniform((uint32_t)v);
-}
-
-__device__ __forceinline__ uint64_t ld_agent64(const uint64_t* p)
-{
-    return __hip_atomic_load(const_cast<uint64_t*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-__device__ __forceinline__ uint32_t ld_agent32(const uint32_t* p)
-{
-    return __hip_atomic_load(const_cast<uint32_t*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-__device__ __forceinline__ uint64_t ld_system64(const uint64_t* p)
-{
-    return __hip_atomic_load(const_cast<uint64_t*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-}
-
-__device__ __forceinline__ uint32_t ld_system32(const uint32_t* p)
-{
-    return __hip_atomic_load(const_cast<uint32_t*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-}
-
-__device__ __forceinline__ void st_agent32(uint32_t* p, uint32_t v)
-{
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-__device__ __forceinline__ void st_agent64(uint64_t* p, uint64_t v)
-{
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-__device__ __forceinline__ bool cas_agent64(uint64_t* p, uint64_t expect, uint64_t want)
-{
-    return __hip_atomic_compare_exchange_strong(p, &expect, want, __ATOMIC_ACQ_REL, __ATOMIC_RELAXED,
-                                                __HIP_MEMORY_SCOPE_AGENT);
-}
 
 // Wave-uniform copy of *p: vector loads (slot memory is written inside the
 // kernel, so it may not go through the scalar cache) broadcast from lane 0.
@@ -2423,6 +3002,18 @@ hipError_t launch_tracks(const WalkArgs& a, bool gauss, bool zref, hipStream_t s
     return hipGetLastError();
 }
 
+// CUs of the current device.
+static uint32_t device_cus()
+{
+    int dev = 0, n = 0;
+    (void)hipGetDevice(&dev);
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) {
+        (void)hipGetLastError();
+        n = 256;
+    }
+    return (uint32_t)n;
+}
+
 // Sorted 16-bit bins that fit in the LDS a workgroup of `fn` may add to its
 // `base` bytes of dynamic LDS without lowering the workgroups per CU that its
 // registers and `base` allow; at most `most`, a multiple of 64, 0 if none.
@@ -2451,32 +3042,48 @@ static uint32_t lds_bins_free(const void* fn, int threads, size_t base, uint32_t
     return cap;
 }
 
-// LDS sorted-bin capacity of distance_kernel<SEG> per (device, base size),
-// found once: the occupancy queries are host calls that do not touch a stream.
-template <int SEG>
-static uint32_t dist_lds_bins(size_t base)
+// LDS sorted-bin capacity of a distance kernel per (device, kernel, base
+// size), found once: the occupancy queries are host calls that do not touch a
+// stream.
+static uint32_t dist_lds_bins(const void* fn, int threads, size_t base, uint32_t most)
 {
     static std::mutex mu;
-    static std::map<std::pair<int, size_t>, uint32_t> memo;
+    static std::map<std::tuple<int, const void*, size_t>, uint32_t> memo;
     int dev = 0;
     (void)hipGetDevice(&dev);
     std::lock_guard<std::mutex> lk(mu);
-    const auto key = std::make_pair(dev, base);
+    const auto key = std::make_tuple(dev, fn, base);
     auto it = memo.find(key);
     if (it != memo.end()) return it->second;
-    const uint32_t cap = lds_bins_free(reinterpret_cast<const void*>(distance_kernel<SEG>), kDistThreads, base,
-                                       (uint32_t)kDistHeld * kDistThreads);
+    const uint32_t cap = lds_bins_free(fn, threads, base, most);
     memo.emplace(key, cap);
     return cap;
 }
 
 template <int SEG>
-static void launch_distance_t(DistArgs a, size_t base, hipStream_t s)
+static void launch_distance_t(DistArgs a, uint32_t n_k_max, uint32_t n_de_max, hipStream_t s)
 {
+    a.colh_off = (n_k_max + 3u) & ~3u;
+    const size_t base = ((size_t)a.colh_off + ((n_de_max + 3u) & ~3u)) * sizeof(uint32_t);
     a.srtl_off = (uint32_t)(base / sizeof(uint32_t));
-    a.srtl_cap = dist_lds_bins<SEG>(base);
+    a.srtl_cap = dist_lds_bins(reinterpret_cast<const void*>(distance_kernel<SEG>), kDistThreads, base,
+                               (uint32_t)kDistHeld * kDistThreads);
     const size_t shmem = base + ((size_t)a.srtl_cap + 1u) / 2u * sizeof(uint32_t);
     hipLaunchKernelGGL(distance_kernel<SEG>, dim3(a.n_props), dim3(kDistThreads), shmem, s, a);
+}
+
+template <int CPL, int NW>
+static void launch_split_t(DistArgs a, uint32_t n_k_max, hipStream_t s)
+{
+    a.piece_off = counter_words(n_k_max);
+    a.diff_off = rows_words(n_k_max);
+    a.base_off = a.diff_off + (uint32_t)(NW * 64 * CPL);
+    a.misc_off = a.base_off + (a.parts > 1u ? 64u * CPL : 0u);
+    a.srtl_off = a.misc_off + (uint32_t)kSplitMisc;
+    const size_t base = (size_t)a.srtl_off * sizeof(uint32_t);
+    a.srtl_cap = dist_lds_bins(reinterpret_cast<const void*>(distance_split_kernel<CPL, NW>), NW * kWave, base, 1u << 15);
+    const size_t shmem = base + ((size_t)a.srtl_cap + 1u) / 2u * sizeof(uint32_t);
+    hipLaunchKernelGGL((distance_split_kernel<CPL, NW>), dim3(a.n_props * a.parts), dim3(NW * kWave), shmem, s, a);
 }
 
 hipError_t launch_distance(const DistArgs& args, uint32_t n_k_max, uint32_t n_de_max, hipStream_t s)
@@ -2486,13 +3093,38 @@ hipError_t launch_distance(const DistArgs& args, uint32_t n_k_max, uint32_t n_de
     if (n_k_max == 0u || n_k_max > PCS_MAX_NK || n_de_max == 0u || n_de_max > PCS_MAX_NDE)
         return hipErrorInvalidValue;
     DistArgs a = args;
-    a.colh_off = (n_k_max + 3u) & ~3u;
-    const size_t base = ((size_t)a.colh_off + ((n_de_max + 3u) & ~3u)) * sizeof(uint32_t);
-    if (n_de_max <= 256) launch_distance_t<1>(a, base, s);
-    else if (n_de_max <= 512) launch_distance_t<2>(a, base, s);
-    else if (n_de_max <= 1024) launch_distance_t<4>(a, base, s);
-    else if (n_de_max <= 2048) launch_distance_t<8>(a, base, s);
-    else launch_distance_t<16>(a, base, s);
+    const uint32_t n_cu = device_cus();
+    a.parts = 1u;
+    // Up to four simulations a CU the rows are split over waves; past that
+    // enough workgroups wait for each other's latency, and the block form's
+    // smaller working set (8 workgroups a CU) wins. Split against block form,
+    // H 1000x500: 300 simulations 126 against 168 us, 700: 173 against 194,
+    // 1,000: 203 both, 2,000: 316 against 270; H 1000x1000 with 73,000 records
+    // each: 61 simulations 166 against 480 us, 3: 88 against 400.
+    if (n_de_max <= 1024u && a.n_props <= 4u * n_cu) {
+        // As many workgroups share a simulation as give every CU one (more
+        // read the slice oftener than they save: 61 simulations by 4 166 us,
+        // by 8 217). Past one simulation a CU, 8 waves let two fit a CU
+        // (500 simulations: 130 us, with 16 waves 165).
+        if (a.scratch)
+            a.parts = std::max(1u, std::min(std::min(kDistMaxParts, n_cu / a.n_props), kDistSlots / a.n_props));
+        const uint32_t cpl = dist_cpl(n_de_max);
+        if (a.n_props <= n_cu) {
+            if (cpl == 4u) launch_split_t<4, 16>(a, n_k_max, s);
+            else if (cpl == 8u) launch_split_t<8, 16>(a, n_k_max, s);
+            else launch_split_t<16, 16>(a, n_k_max, s);
+        } else {
+            if (cpl == 4u) launch_split_t<4, 8>(a, n_k_max, s);
+            else if (cpl == 8u) launch_split_t<8, 8>(a, n_k_max, s);
+            else launch_split_t<16, 8>(a, n_k_max, s);
+        }
+        return hipGetLastError();
+    }
+    if (n_de_max <= 256) launch_distance_t<1>(a, n_k_max, n_de_max, s);
+    else if (n_de_max <= 512) launch_distance_t<2>(a, n_k_max, n_de_max, s);
+    else if (n_de_max <= 1024) launch_distance_t<4>(a, n_k_max, n_de_max, s);
+    else if (n_de_max <= 2048) launch_distance_t<8>(a, n_k_max, n_de_max, s);
+    else launch_distance_t<16>(a, n_k_max, n_de_max, s);
     return hipGetLastError();
 }
 

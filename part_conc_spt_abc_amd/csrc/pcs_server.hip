@@ -115,6 +115,7 @@ struct Group {
     uint32_t *d_vframes = nullptr, *d_vparticles = nullptr, *d_vprop = nullptr;
     uint32_t* d_vtile[kClasses] = {};
     uint32_t* d_count = nullptr;
+    DistScratch* d_dscratch = nullptr;
     // pinned host staging (uploads) and results (written by the distance kernel)
     DevProp* h_props = nullptr;
     uint32_t *h_vframes = nullptr, *h_vparticles = nullptr, *h_vprop = nullptr;
@@ -215,6 +216,8 @@ hipError_t group_alloc(Group& g, uint32_t max_props, uint32_t max_videos)
     if (e == hipSuccess) e = dmalloc(&g.d_vprop, max_videos);
     for (int k = 0; k < kClasses && e == hipSuccess; ++k) e = dmalloc(&g.d_vtile[k], max_videos + 1);
     if (e == hipSuccess) e = dmalloc(&g.d_count, max_props);
+    if (e == hipSuccess) e = dmalloc(&g.d_dscratch, 1);
+    if (e == hipSuccess) e = hipMemset(g.d_dscratch, 0, sizeof(DistScratch));
     if (e == hipSuccess) e = hmalloc(&g.h_props, max_props);
     if (e == hipSuccess) e = hmalloc(&g.h_vframes, max_videos);
     if (e == hipSuccess) e = hmalloc(&g.h_vparticles, max_videos);
@@ -230,7 +233,7 @@ hipError_t group_alloc(Group& g, uint32_t max_props, uint32_t max_videos)
 void group_free(Group& g)
 {
     if (g.stream) hipStreamSynchronize(g.stream);
-    void* dev[] = {g.d_props, g.d_vframes, g.d_vparticles, g.d_vprop, g.d_count};
+    void* dev[] = {g.d_props, g.d_vframes, g.d_vparticles, g.d_vprop, g.d_count, g.d_dscratch};
     for (void* p : dev)
         if (p) hipFree(p);
     void* host[] = {g.h_props, g.h_vframes, g.h_vparticles, g.h_vprop, g.h_dist, g.h_exact, g.h_tracks, g.h_status};
@@ -339,6 +342,7 @@ int launch_group(pcs_server* s, Group& g, std::vector<Pending>& batch, std::vect
         d.exact = g.h_exact;
         d.tracks = g.h_tracks;
         d.status = g.h_status;
+        d.scratch = g.d_dscratch;
         e = launch_distance(d, n_k_max, n_de_max, st);
     }
     if (e == hipSuccess) e = hipEventRecord(g.done, st);
@@ -825,14 +829,14 @@ int pcs_server_add_system(pcs_server* s, const pcs_system* sys, const uint32_t* 
     std::lock_guard<std::mutex> lk(s->mu);
     if (s->systems.size() >= kMaxSystems) return set_error(PCS_EINVAL, "more than %u systems", kMaxSystems);
     std::vector<uint32_t> sat;
-    uint32_t maxrow = 0;
-    build_sat(obs_hist, sys->n_k, sys->n_de, sat, maxrow);
+    uint32_t maxrow = 0, most = 0;
+    build_sat(obs_hist, sys->n_k, sys->n_de, sat, maxrow, most);
     SysEntry ent;
     ent.sys = *sys;
     hipError_t e = hipSetDevice(s->device);
     if (e == hipSuccess) e = dmalloc(&ent.d_sat, sat.size());
     if (e == hipSuccess) e = hipMemcpy(ent.d_sat, sat.data(), sat.size() * 4, hipMemcpyHostToDevice);
-    const DevSys d = make_devsys(*sys, maxrow, ent.d_sat);
+    const DevSys d = make_devsys(*sys, maxrow, most, ent.d_sat);
     const uint32_t id = (uint32_t)s->systems.size();
     if (e == hipSuccess) e = hipMemcpy(s->d_sys + id, &d, sizeof(DevSys), hipMemcpyHostToDevice);
     if (e != hipSuccess) {
