@@ -799,16 +799,21 @@ __device__ __forceinline__ void walk_tile_coop(const DevProp& pr, const DevSys& 
 
 // Tile t of a batch plan: the video owning it is the largest v with
 // vtile[v] <= t (wave-uniform binary search).
-template <int PPL, bool GAUSS, bool ZREF, bool TRACKS>
-__device__ __forceinline__ void process_tile(const WalkArgs& a, uint32_t t, Stage& st, const float2* tab,
-                                             uint32_t s0, uint32_t s1)
+__device__ __forceinline__ uint32_t tile_video(const WalkArgs& a, uint32_t t)
 {
     uint32_t lo = 0u, hi = a.n_videos;
     while (hi - lo > 1u) {
         const uint32_t mid = (lo + hi) >> 1;
         if (a.vtile[mid] <= t) lo = mid; else hi = mid;
     }
-    const uint32_t v = lo;
+    return lo;
+}
+
+template <int PPL, bool GAUSS, bool ZREF, bool TRACKS>
+__device__ __forceinline__ void process_tile(const WalkArgs& a, uint32_t t, Stage& st, const float2* tab,
+                                             uint32_t s0, uint32_t s1)
+{
+    const uint32_t v = tile_video(a, t);
     const uint32_t P = a.vprop[v];
     const DevProp& pr = a.props[P];
     st.rec = pr.rec;
@@ -891,6 +896,298 @@ __device__ __forceinline__ bool cas_agent64(uint64_t* p, uint64_t expect, uint64
 {
     return __hip_atomic_compare_exchange_strong(p, &expect, want, __ATOMIC_ACQ_REL, __ATOMIC_RELAXED,
                                                 __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// ------------------------------------------------------ walk of few tiles
+//
+// A tile walked by one wave takes as long as that wave's instruction stream:
+// with few tiles on the GPU a wave is alone on its SIMD and issues one
+// instruction per 4 to 8 cycles (0.25 us a frame), a third of what the SIMD
+// can. Here a workgroup of 11 waves walks a tile. What depends on the frame
+// before is little - the positions, and the open tracks - and goes to three
+// waves: one steps x and y, one z, one follows the tracks. The other eight make
+// the unit normals, a 4-step chunk each, which depend on no earlier frame.
+// In round i the producers make chunks 8i..8i+7, the movers step the 32 frames
+// of round i - 1 and leave each lane's window tests as a 32-bit history, and
+// the tracker takes round i - 2's histories; one barrier a round. Every value
+// and its order are walk_tile's. Bound by the serial waves' dependent
+// instructions, about 70 cycles a frame in each mover and 130 in the tracker;
+// a producer takes about 70. A lone simulation of 20 tiles x 1,000 frames:
+// 329 us a wave a tile, 74 us so.
+// LDS: the angle tables, normals of two rounds, squared steps of three (the
+// tracker is a round later), histories of two, the tracker's record stage:
+// 79 KB, two workgroups a CU (97 KB and one with Gaussian detection).
+constexpr int kGrpProd = 8;
+constexpr int kGrpThreads = (3 + kGrpProd) * kWave;
+constexpr uint32_t kGrpSteps = 4u * kGrpProd;
+constexpr uint32_t kGrpStage = 768;
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+// bits = 2 bits + (lane's bit of m): the lane's history of a window test.
+__device__ __forceinline__ void push_bit(uint32_t& bits, uint64_t m)
+{
+    uint64_t carry;
+    asm("v_addc_co_u32_e64 %0, %1, %0, %0, %2" : "+v"(bits), "=s"(carry) : "s"(m));
+}
+
+// OR over the wave (data-parallel-primitive moves, as wave_incl_scan below).
+__device__ __forceinline__ uint32_t wave_or(uint32_t v)
+{
+    int x = (int)v;
+    x |= __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false);
+    x |= __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false);
+    x |= __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false);
+    x |= __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false);
+    x |= __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);
+    x |= __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);
+    return (uint32_t)__builtin_amdgcn_readlane(x, 63);
+}
+
+template <bool GAUSS, bool ZREF>
+__global__ __launch_bounds__(kGrpThreads) void walk_group_kernel(WalkArgs a)
+{
+    constexpr bool ZBOX = !ZREF;
+    constexpr uint32_t B = GAUSS ? 3u : 2u;
+    constexpr uint32_t NB = kGrpProd * kWave;  // lane entries of a round's chunks
+    extern __shared__ __align__(16) uint32_t grp_lds[];
+    float* tabf = reinterpret_cast<float*>(grp_lds);
+    float2* xy = reinterpret_cast<float2*>(tabf + kAngleTabFloats);  // [2][chunk][step][lane]
+    f32x4* zz = reinterpret_cast<f32x4*>(xy + 2 * 4 * NB);           // [2][chunk][lane], a step a component
+    f32x4* rr = zz + 2 * NB;                                         // [3][chunk][lane]
+    uint32_t* hist = reinterpret_cast<uint32_t*>(rr + 3 * NB);       // [2][x and y | z][lane]
+    uint32_t* stage = hist + 4 * kWave;
+    u32x4* wd = reinterpret_cast<u32x4*>(stage + kGrpStage);         // Gaussian detection: [2][chunk][lane]
+
+    load_angle_table(tabf);
+    __syncthreads();
+    const float2* tab = reinterpret_cast<const float2*>(tabf);
+    const uint64_t seed = *a.seed;
+    const uint32_t wave = uniform(threadIdx.x / kWave), lane = lane_id();
+
+    for (uint32_t t = a.tile_lo + blockIdx.x; t < a.tile_hi; t += gridDim.x) {
+        const uint32_t v = uniform(tile_video(a, t));
+        const uint32_t P = uniform(a.vprop[v]);
+        const DevProp& pr = a.props[P];
+        const DevSys& sy = a.sys[pr.sys_id];
+        const uint32_t N = uniform(a.vparticles[v]), F = uniform(a.vframes[v]);
+        const uint32_t video = uniform(v - pr.first_video), sim = uniform(pr.sim_id);
+        const uint32_t k0 = uniform((uint32_t)seed ^ pr.key0), k1 = uniform((uint32_t)(seed >> 32) ^ pr.key1);
+        const uint32_t id = (t - uniform(a.vtile[v])) * (uint32_t)kWave + lane;
+        const WalkConsts K = walk_consts<GAUSS, ZREF>(sy);
+        const uint32_t steps = F > 0u ? F - 1u : 0u;
+        const uint32_t nr = (steps + kGrpSteps - 1u) / kGrpSteps;
+        // Every role runs nr + 2 rounds with one barrier each.
+        if (wave >= 3u) {
+            const uint32_t j = wave - 3u;
+            for (uint32_t it = 0; it < nr + 2u; ++it) {
+                const uint32_t c = it * kGrpProd + j;
+                if (4u * c < steps) {
+                    const uint32_t e = (it & 1u) * NB + j * kWave + lane;
+                    const U4 b0 = philox10(B * c + 1u, id, video, sim, k0, k1);
+                    const U4 b1 = philox10(B * c + 2u, id, video, sim, k0, k1);
+                    const uint32_t w[8] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
+                    float2* xs = xy + ((it & 1u) * NB + j * kWave) * 4u + lane;
+                    f32x4 r2, nz;
+#pragma unroll
+                    for (int p = 0; p < 6; ++p) {
+                        float d0, d1, y;
+                        bm_pair(w[p], w[6 + p / 4], p, tab, d0, d1, y);
+                        if (p < 4) {
+                            xs[p * kWave] = float2{d0, d1};
+                            r2[p] = y;
+                        } else {
+                            nz[2 * (p - 4)] = d0;
+                            nz[2 * (p - 4) + 1] = d1;
+                        }
+                    }
+                    zz[e] = nz;
+                    rr[(it % 3u) * NB + j * kWave + lane] = r2;
+                    if (GAUSS) {
+                        const U4 b2 = philox10(B * c + 3u, id, video, sim, k0, k1);
+                        wd[e] = u32x4{b2.x, b2.y, b2.z, b2.w};
+                    }
+                }
+                __syncthreads();
+            }
+            continue;
+        }
+        __builtin_amdgcn_s_setprio(3);
+        Particle q;
+        q.id = id;
+        init_particle<GAUSS, ZREF>(q, N, video, sim, k0, k1, pr, K);
+        if (wave == 0u) {
+            for (uint32_t it = 0; it < nr + 2u; ++it) {
+                if (it >= 1u && it <= nr) {
+                    const uint32_t n = min(kGrpSteps, steps - (it - 1u) * kGrpSteps);
+                    const float2* xs = xy + ((it - 1u) & 1u) * NB * 4u + lane;
+                    uint32_t bits = 0u;
+                    auto step = [&](float2 d) {
+                        q.x = fract_box(__builtin_fmaf(q.sx, d.x, q.x));
+                        q.y = fract_box(__builtin_fmaf(q.sy, d.y, q.y));
+                        push_bit(bits, ballot(q.x <= K.wx) & ballot(q.y <= K.wy));
+                    };
+                    if (n == kGrpSteps) {
+                        float2 d[8], e[8];
+#pragma unroll
+                        for (int s = 0; s < 8; ++s) d[s] = xs[s * kWave];
+#pragma unroll
+                        for (uint32_t s0 = 0; s0 < kGrpSteps; s0 += 8u) {
+                            if (s0 + 8u < kGrpSteps) {
+#pragma unroll
+                                for (int s = 0; s < 8; ++s) e[s] = xs[(s0 + 8u + s) * kWave];
+                            }
+#pragma unroll
+                            for (int s = 0; s < 8; ++s) {
+                                step(d[s]);
+                                d[s] = e[s];
+                            }
+                        }
+                    } else {
+                        for (uint32_t s = 0; s < n; ++s) step(xs[s * kWave]);
+                        bits <<= kGrpSteps - n;  // n >= 1
+                    }
+                    hist[((it - 1u) & 1u) * 2u * kWave + lane] = bits;
+                }
+                __syncthreads();
+            }
+        } else if (wave == 1u) {
+            for (uint32_t it = 0; it < nr + 2u; ++it) {
+                if (it >= 1u && it <= nr) {
+                    const uint32_t n = min(kGrpSteps, steps - (it - 1u) * kGrpSteps);
+                    const uint32_t e = ((it - 1u) & 1u) * NB + lane;
+                    uint32_t bits = 0u;
+                    f32x4 nz = zz[e];
+                    u32x4 w = GAUSS ? wd[e] : u32x4{0u, 0u, 0u, 0u};
+#pragma unroll
+                    for (uint32_t j = 0; j < (uint32_t)kGrpProd; ++j) {
+                        if (4u * j >= n) break;
+                        f32x4 nz1 = nz;
+                        u32x4 w1 = w;
+                        if (j + 1u < (uint32_t)kGrpProd) {  // chunks past the last: read, not used
+                            nz1 = zz[e + (j + 1u) * kWave];
+                            if (GAUSS) w1 = wd[e + (j + 1u) * kWave];
+                        }
+#pragma unroll
+                        for (uint32_t s = 0; s < 4u; ++s) {
+                            if (4u * j + s >= n) break;
+                            if (ZBOX) q.z = fract_box(__builtin_fmaf(q.sz, nz[s], q.z));
+                            else q.z = wrap_reflect(__builtin_fmaf(q.sz, nz[s], q.z), K.hz);
+                            const bool cz = GAUSS ? gauss_detect(ZBOX ? q.z - 0.5f : q.z, K.cg, w[s])
+                                                  : (ZBOX ? q.z <= q.wz : __builtin_fabsf(q.z) <= q.wz);
+                            push_bit(bits, ballot(cz));
+                        }
+                        nz = nz1;
+                        w = w1;
+                    }
+                    if (n < kGrpSteps) bits <<= kGrpSteps - n;
+                    hist[(((it - 1u) & 1u) * 2u + 1u) * kWave + lane] = bits;
+                }
+                __syncthreads();
+            }
+        } else {
+            Stage st;
+            st.buf = stage;
+            st.cap = kGrpStage;
+            st.cnt = 0u;
+            st.rec = pr.rec;
+            st.slice_cap = pr.rec_cap;
+            st.counter = a.rec_count + P;
+            // A lane's frame bits, the round's first in the top one, and those
+            // of the frames before it, the last in bit 0 of `prev`. Tracks
+            // start where the window is entered and end where it is left, and
+            // whether one of at least kmin frames ends is kmin bits in a row:
+            // bit operations on the whole round. (Up to 32 bits; the closing
+            // code tests the length itself.) What is left a frame is the sum
+            // of squared steps (0 again at a start; a lane outside the window
+            // sums steps that no track takes), and the frames in which some
+            // lane's track closes.
+            const uint32_t on = q.active ? ~0u : 0u;  // no tracks on lanes without a particle
+            const uint32_t run = min(K.kmin, 32u);
+            uint32_t prev = q.det0 ? on & 1u : 0u;
+            for (uint32_t it = 0; it < nr + 2u; ++it) {
+                if (it >= 2u) {
+                    const uint32_t n = min(kGrpSteps, steps - (it - 2u) * kGrpSteps);
+                    const uint32_t h = (it & 1u) * 2u * kWave + lane;
+                    const uint32_t bits = hist[h] & hist[h + kWave] & on;  // 0 past frame n
+                    const uint64_t both = (uint64_t)prev << 32 | bits;
+                    uint64_t row = both;  // bit set: `have` bits in a row end there
+                    uint32_t have = 1u;
+                    for (; 2u * have <= run; have *= 2u) row &= row >> have;
+                    row &= row >> (run - have);
+                    const uint32_t starts = bits & ~(uint32_t)(both >> 1);
+                    const uint32_t ends = (uint32_t)(row >> 1) & ~bits & ~0u << (kGrpSteps - n);
+                    prev = (uint32_t)(both >> (kGrpSteps - n));
+                    // A lane's first close of the round takes its sum aside as
+                    // the frames go by, and all lanes' are staged after them;
+                    // the few others are staged in their frame.
+                    const uint32_t first = ends != 0u ? 0x80000000u >> __builtin_clz(ends) : 0u;
+                    const uint32_t others = ends & ~first;
+                    const uint32_t any = wave_or(others);
+                    uint32_t de_first = 0u;
+                    // Stage the track of the lanes of `end` that closes at
+                    // frame f1 - 1 with the sum de: it began at the frame after
+                    // its last start bit, or at q.ts before the round.
+                    auto close = [&](bool end, uint32_t f1, float de) {
+                        const uint32_t was = f1 > 1u ? starts >> (kGrpSteps + 1u - f1) : 0u;
+                        const int32_t ts = was ? (int32_t)(f1 - 1u) - __builtin_ctz(was) : q.ts;
+                        const uint64_t m = ballot(end && ts <= (int32_t)(f1 - K.kmin));
+                        const uint32_t pos = st.cnt + 2u * mbcnt64(m);
+                        if (__builtin_amdgcn_inverse_ballot_w64(m)) {
+                            st.buf[pos] = f1 - (uint32_t)ts;
+                            st.buf[pos + 1u] = __float_as_uint(q.sig2 * de);
+                        }
+                        st.cnt += 2u * (uint32_t)__builtin_popcountll(m);
+                    };
+                    const f32x4* rs = rr + ((it - 2u) % 3u) * NB + lane;
+                    f32x4 r2 = rs[0];
+                    // One frame: a lane whose first close it is takes the sum
+                    // aside; then the sum goes on, from 0 at a start.
+                    auto frame = [&](uint32_t stay, uint32_t fb, int s, float step2) {
+                        const uint32_t at = (uint32_t)__builtin_amdgcn_sbfe((int)fb, 31u - s, 1u);
+                        const uint32_t keep = (uint32_t)__builtin_amdgcn_sbfe((int)stay, 31u - s, 1u);
+                        de_first = (__float_as_uint(q.de) & at) | (de_first & ~at);
+                        q.de = __uint_as_float(__float_as_uint(q.de + step2) & keep);
+                    };
+                    // Two chunks a turn, the path without other closes laid
+                    // out straight: a lone wave loses 40 cycles or more to a
+                    // branch it takes.
+#pragma unroll 2
+                    for (uint32_t j = 0; 4u * j < n; ++j) {
+                        const f32x4 r1 = rs[min(j + 1u, (uint32_t)kGrpProd - 1u) * kWave];
+                        if (__builtin_expect(4u * j + 4u > n, 0)) {  // frames past the last add nothing
+#pragma unroll
+                            for (uint32_t s = 1; s < 4u; ++s) r2[s] = 4u * j + s < n ? r2[s] : 0.0f;
+                        }
+                        const uint32_t some = any << 4u * j >> 28;
+                        const uint32_t stay = ~starts << 4u * j, fb = first << 4u * j;
+                        if (__builtin_expect(some != 0u, 0)) {
+                            if (st.cnt + 8u * kWave > st.cap) stage_flush_binned(st, K.bs);
+                            for (int s = 0; s < 4; ++s) {
+                                if (some & 8u >> s)
+                                    close((others << 4u * j & 0x80000000u >> s) != 0u, 4u * j + (uint32_t)s + 1u, q.de);
+                                const float step2 = s == 0 ? r2[0] : (s == 1 ? r2[1] : (s == 2 ? r2[2] : r2[3]));
+                                frame(stay << s, fb << s, 0, step2);
+                            }
+                        } else {
+#pragma unroll
+                            for (int s = 0; s < 4; ++s) frame(stay, fb, s, r2[s]);
+                        }
+                        r2 = r1;
+                    }
+                    if (st.cnt + 2u * kWave > st.cap) stage_flush_binned(st, K.bs);
+                    close(first != 0u, (uint32_t)__builtin_clz(first | 1u) + 1u, __uint_as_float(de_first));
+                    if (starts != 0u) q.ts = (int32_t)kGrpSteps - __builtin_ctz(starts);
+                    q.ts -= (int32_t)n;  // the round's last frame becomes frame 0
+                }
+                __syncthreads();
+            }
+            close_open_tracks<false>(q, ballot(q.active), ballot((prev & 1u) != 0u), K, st);
+            stage_flush_binned(st, K.bs);
+        }
+        __builtin_amdgcn_s_setprio(0);
+    }
 }
 
 // --------------------------------------------------------------- distance
@@ -1376,7 +1673,6 @@ void distance_kernel(DistArgs a)
 
 // ------------------------------------------- distance of few simulations
 
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4u __attribute__((ext_vector_type(4), aligned(4)));  // a quad at any record
 
 // Rows with at most this many records enter a lane's columns by comparison,
@@ -2951,6 +3247,18 @@ hipError_t launch_reset(uint32_t* rec_count, uint32_t n, uint32_t* tile_counter,
     return hipGetLastError();
 }
 
+// CUs of the current device.
+static uint32_t device_cus()
+{
+    int dev = 0, n = 0;
+    (void)hipGetDevice(&dev);
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) {
+        (void)hipGetLastError();
+        n = 256;
+    }
+    return (uint32_t)n;
+}
+
 template <int PPL, bool PERSIST, bool GAUSS, bool ZREF>
 static hipError_t launch_walk_t(const WalkArgs& a, int wpg, uint32_t grid, hipStream_t s)
 {
@@ -2969,10 +3277,33 @@ static hipError_t launch_walk_m(const WalkArgs& a, int wpg, uint32_t grid, bool 
                 : launch_walk_t<PPL, PERSIST, false, false>(a, wpg, grid, s);
 }
 
+template <bool GAUSS, bool ZREF>
+static hipError_t launch_group_t(const WalkArgs& a, uint32_t grid, hipStream_t s)
+{
+    (void)hipGetLastError();  // report only this launch's error
+    constexpr size_t words = kAngleTabFloats + (size_t)kGrpProd * kWave * (2 * 8 + 2 * 4 + 3 * 4 + (GAUSS ? 2 * 4 : 0)) +
+                             4 * kWave + kGrpStage;
+    hipLaunchKernelGGL((walk_group_kernel<GAUSS, ZREF>), dim3(grid), dim3(kGrpThreads), words * sizeof(uint32_t), s, a);
+    return hipGetLastError();
+}
+
 hipError_t launch_walk(const WalkArgs& a, int ppl, int wpg, bool persistent, uint32_t grid_groups,
                        bool gauss, bool zref, hipStream_t s)
 {
     if (a.tile_hi <= a.tile_lo) return hipSuccess;
+    // Few tiles: a workgroup each, as long as that beats a wave each. At 1,000
+    // frames, group against wave: 4 tiles (500 frames) 41 against 205 us, 379
+    // 92 against 370, 1,510 270 against 500, 3,005 532 against 645, 4,520 770
+    // against 755; Gaussian detection at 2,000 frames 1,506 tiles 735 against
+    // 1,180, 3,005 1,420 against 1,460, 6,002 2,750 against 1,800. (A range
+    // planned on the device is not known here, and tiles of 128 particles are
+    // not the group's.)
+    const uint32_t n_cu = device_cus();
+    if (ppl == 1 && !a.tile_total && a.tile_hi - a.tile_lo <= (gauss ? 11u : 14u) * n_cu) {
+        const uint32_t grid = std::min(a.tile_hi - a.tile_lo, (gauss ? 1u : 2u) * n_cu);
+        if (gauss) return zref ? launch_group_t<true, true>(a, grid, s) : launch_group_t<true, false>(a, grid, s);
+        return zref ? launch_group_t<false, true>(a, grid, s) : launch_group_t<false, false>(a, grid, s);
+    }
     uint32_t grid = grid_groups;
     if (!persistent) {
         const uint32_t n = a.tile_hi - a.tile_lo;
@@ -3000,18 +3331,6 @@ hipError_t launch_tracks(const WalkArgs& a, bool gauss, bool zref, hipStream_t s
     else
         hipLaunchKernelGGL((walk_kernel<1, false, false, false, true>), dim3(grid), dim3(256), shmem, s, a);
     return hipGetLastError();
-}
-
-// CUs of the current device.
-static uint32_t device_cus()
-{
-    int dev = 0, n = 0;
-    (void)hipGetDevice(&dev);
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0) {
-        (void)hipGetLastError();
-        n = 256;
-    }
-    return (uint32_t)n;
 }
 
 // Sorted 16-bit bins that fit in the LDS a workgroup of `fn` may add to its
