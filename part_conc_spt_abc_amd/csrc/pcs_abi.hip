@@ -143,6 +143,9 @@ struct pcs_ctx {
     // The caller's handle plus one per live batch: pcs_close drops the
     // caller's, and the context is freed when its last batch is destroyed.
     std::atomic<int> refs{1};
+    // pcs_simulate's batch, kept from call to call while it is small (making
+    // and freeing one costs 150 us of allocations); pcs_close gives it back.
+    pcs_batch* oneshot = nullptr;
 };
 
 struct pcs_batch {
@@ -160,10 +163,20 @@ struct pcs_batch {
     // device
     DevProp* d_props = nullptr;
     uint32_t *d_vframes = nullptr, *d_vparticles = nullptr, *d_vprop = nullptr, *d_vtile = nullptr;
-    uint32_t *d_rec = nullptr, *d_srt = nullptr, *d_count = nullptr, *d_tracks = nullptr, *d_tile_counter = nullptr;
+    uint32_t *d_rec = nullptr, *d_srt = nullptr, *d_count = nullptr, *d_tile_counter = nullptr;
+    // Results: written by the distance kernel straight into pinned host memory
+    // for up to kHostResults simulations (a read is then one wait; copying
+    // the arrays back cost 60 us), into device memory above.
+    bool host_res = false;
+    uint32_t* d_tracks = nullptr;
     double* d_dist = nullptr;
     uint64_t* d_exact = nullptr;
     int32_t* d_status = nullptr;
+    // dense histograms on their way to the caller: device chunk and pinned
+    // staging, kept up to kHistKeep bytes each
+    uint32_t *d_hist = nullptr, *h_hist = nullptr;
+    size_t cap_hist = 0;
+    bool plan_ran = false;  // the present plan has run once (the graph pays from the second run on)
     uint64_t* d_seed = nullptr;
     uint64_t* h_seed = nullptr;  // pinned
     size_t cap_props = 0, cap_videos = 0, cap_arena = 0;
@@ -234,6 +247,10 @@ int dev_alloc(T** p, size_t n)
     return PCS_OK;
 }
 
+constexpr uint32_t kHostResults = 4096;
+constexpr size_t kHistKeep = 16u << 20;     // bytes
+constexpr uint64_t kOneshotKeep = 4u << 20;  // records of a kept pcs_simulate batch
+
 #define PCS_HIP(call)                                         \
     do {                                                      \
         const hipError_t e_ = (call);                         \
@@ -246,12 +263,56 @@ int dev_alloc(T** p, size_t n)
         if (r_ != PCS_OK) return r_;    \
     } while (0)
 
+void free_results(pcs_batch* b)
+{
+    void* ptrs[] = {b->d_tracks, b->d_dist, b->d_exact, b->d_status};
+    for (void* q : ptrs)
+        if (q) b->host_res ? hipHostFree(q) : hipFree(q);
+    b->d_tracks = nullptr;
+    b->d_dist = nullptr;
+    b->d_exact = nullptr;
+    b->d_status = nullptr;
+}
+
+// Result arrays of n simulations (the stream is idle).
+int alloc_results(pcs_batch* b, uint32_t n)
+{
+    free_results(b);
+    b->host_res = n <= kHostResults;
+    if (!b->host_res) {
+        PCS_TRY(dev_alloc(&b->d_tracks, n));
+        PCS_TRY(dev_alloc(&b->d_dist, n));
+        PCS_TRY(dev_alloc(&b->d_exact, n));
+        return dev_alloc(&b->d_status, n);
+    }
+    const size_t m = n ? n : 1;
+    hipError_t e = hipHostMalloc((void**)&b->d_tracks, m * 4u, hipHostMallocDefault);
+    if (e == hipSuccess) e = hipHostMalloc((void**)&b->d_dist, m * 8u, hipHostMallocDefault);
+    if (e == hipSuccess) e = hipHostMalloc((void**)&b->d_exact, m * 8u, hipHostMallocDefault);
+    if (e == hipSuccess) e = hipHostMalloc((void**)&b->d_status, m * 4u, hipHostMallocDefault);
+    if (e != hipSuccess) return set_error(PCS_ENOMEM, "hipHostMalloc (results of %u simulations): %s", n, hipGetErrorString(e));
+    return PCS_OK;
+}
+
+// Copies n results to the host: the stream is idle when they are already there.
+template <typename T>
+int fetch_results(pcs_batch* b, T* out, const T* res)
+{
+    if (b->host_res) {
+        std::copy(res, res + b->n_props, out);
+        return PCS_OK;
+    }
+    PCS_HIP(hipMemcpyAsync(out, res, b->n_props * sizeof(T), hipMemcpyDeviceToHost, b->stream));
+    return PCS_OK;
+}
+
 void destroy_graph(pcs_batch* b)
 {
     if (b->gexec) hipGraphExecDestroy(b->gexec);
     if (b->graph) hipGraphDestroy(b->graph);
     b->gexec = nullptr;
     b->graph = nullptr;
+    b->plan_ran = false;
 }
 
 int check_tuning(const pcs_tuning& t)
@@ -441,6 +502,7 @@ int enqueue_plain(pcs_batch* b, const std::vector<uint32_t>* subset, bool stream
 int capture_graph_once(pcs_batch* b, bool events)
 {
     destroy_graph(b);
+    b->graph_events = false;
     PCS_HIP(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
     const int r = enqueue_batched(b, events);
     hipGraph_t g = nullptr;
@@ -468,16 +530,26 @@ bool same_tune(const pcs_tuning& a, const pcs_tuning& b) { return std::memcmp(&a
 // the next run restores them.
 int rerun_overflows(pcs_batch* b)
 {
-    std::vector<int32_t> st(b->n_props);
-    std::vector<uint32_t> cnt(b->n_props);
-    PCS_HIP(hipMemcpyAsync(st.data(), b->d_status, b->n_props * 4, hipMemcpyDeviceToHost, b->stream));
-    PCS_HIP(hipMemcpyAsync(cnt.data(), b->d_count, b->n_props * 4, hipMemcpyDeviceToHost, b->stream));
-    PCS_HIP(hipStreamSynchronize(b->stream));
+    std::vector<int32_t> st_h;
+    std::vector<uint32_t> cnt_h;
+    const int32_t* st = b->d_status;
+    const uint32_t* cnt = b->d_tracks;  // an overflowed slice's count
+    if (!b->host_res) {
+        st_h.resize(b->n_props);
+        cnt_h.resize(b->n_props);
+        PCS_TRY(fetch_results(b, st_h.data(), b->d_status));
+        PCS_TRY(fetch_results(b, cnt_h.data(), b->d_tracks));
+        PCS_HIP(hipStreamSynchronize(b->stream));
+        st = st_h.data();
+        cnt = cnt_h.data();
+    }
     std::vector<uint32_t> over;
+    std::vector<uint32_t> size;
     uint64_t need = 0;
     for (uint32_t i = 0; i < b->n_props; ++i)
         if (st[i] == PCS_EOVERFLOW) {
             over.push_back(i);
+            size.push_back(cnt[i]);
             need += cnt[i];
         }
     b->reruns = (uint32_t)over.size();
@@ -498,8 +570,8 @@ int rerun_overflows(pcs_batch* b)
         const uint32_t P = over[k];
         dp[k].rec = b->d_rec2 + off;
         dp[k].srt = b->d_srt2 + off;
-        dp[k].rec_cap = cnt[P];
-        off += cnt[P];
+        dp[k].rec_cap = size[k];
+        off += size[k];
         PCS_HIP(hipMemcpyAsync(b->d_props + P, &dp[k], sizeof(DevProp), hipMemcpyHostToDevice, b->stream));
         PCS_HIP(hipMemsetAsync(b->d_count + P, 0, 4, b->stream));
     }
@@ -715,6 +787,11 @@ void ctx_release(pcs_ctx* c)
 int pcs_close(pcs_ctx* c)
 {
     if (!c) return PCS_OK;
+    if (c->oneshot) {
+        pcs_batch* b = c->oneshot;
+        c->oneshot = nullptr;
+        pcs_batch_destroy(b);
+    }
     ctx_release(c);
     return PCS_OK;
 }
@@ -787,11 +864,13 @@ int pcs_batch_destroy(pcs_batch* b)
     if (b->wstream) hipStreamSynchronize(b->wstream);
     destroy_graph(b);
     void* ptrs[] = {b->d_props, b->d_vframes, b->d_vparticles, b->d_vprop, b->d_vtile, b->d_rec, b->d_srt,
-                    b->d_rec2, b->d_srt2, b->d_count, b->d_tracks, b->d_tile_counter, b->d_dist, b->d_exact, b->d_status,
+                    b->d_rec2, b->d_srt2, b->d_count, b->d_tile_counter, b->d_hist,
                     b->d_seed, b->d_in, b->d_theta_pop, b->d_cumw, b->d_theta_new, b->d_totals, b->d_wpop,
                     b->d_xn, b->d_xo, b->d_wsum, b->d_part, b->d_dscratch};
     for (void* p : ptrs)
         if (p) hipFree(p);
+    free_results(b);
+    if (b->h_hist) hipHostFree(b->h_hist);
     if (b->h_seed) hipHostFree(b->h_seed);
     for (hipEvent_t& e : b->ev)
         if (e) hipEventDestroy(e);
@@ -877,10 +956,7 @@ int pcs_batch_load(pcs_batch* b, const pcs_proposal* props, uint32_t n, const ui
         b->cap_props = 0;
         PCS_TRY(dev_alloc(&b->d_props, n));
         PCS_TRY(dev_alloc(&b->d_count, n));
-        PCS_TRY(dev_alloc(&b->d_tracks, n));
-        PCS_TRY(dev_alloc(&b->d_dist, n));
-        PCS_TRY(dev_alloc(&b->d_exact, n));
-        PCS_TRY(dev_alloc(&b->d_status, n));
+        PCS_TRY(alloc_results(b, n));
         b->cap_props = n;
     }
     if (n_videos + 1 > b->cap_videos) {
@@ -946,10 +1022,15 @@ int pcs_batch_run(pcs_batch* b, uint64_t seed, int mode)
     PCS_HIP(hipMemcpyAsync(b->d_seed, b->h_seed, sizeof(uint64_t), hipMemcpyHostToDevice, b->stream));
     b->reruns = 0;
     if (mode == PCS_MODE_BATCHED) {
-        if (!b->gexec || !same_tune(b->graph_tune, c->tune)) PCS_TRY(capture_graph(b));
+        // Capturing the graph pays when the same plan runs again: the first
+        // run launches the three kernels themselves (15 us less).
+        const bool direct = !b->gexec && !b->plan_ran;
+        if (!direct && (!b->gexec || !same_tune(b->graph_tune, c->tune))) PCS_TRY(capture_graph(b));
         if (!b->graph_events) PCS_HIP(hipEventRecord(b->ev[0], b->stream));
-        PCS_HIP(hipGraphLaunch(b->gexec, b->stream));
+        if (direct) PCS_TRY(enqueue_batched(b, false));
+        else PCS_HIP(hipGraphLaunch(b->gexec, b->stream));
         if (!b->graph_events) PCS_HIP(hipEventRecord(b->ev[3], b->stream));
+        b->plan_ran = true;
     } else if (mode == PCS_MODE_BATCHED_DIRECT) {
         PCS_TRY(enqueue_batched(b, true));
     } else {
@@ -1006,6 +1087,66 @@ int pcs_batch_overflow_reruns(pcs_batch* b, uint32_t* n)
     return PCS_OK;
 }
 
+// Dense histograms, formed from the records in chunks of proposals. They come
+// back through pinned staging, copied out while the next piece is on its way:
+// copies of megabytes into pageable memory took 0.6 to 4 ms for 2 MB.
+static int read_hist(pcs_batch* b, uint32_t* hist_out)
+{
+    pcs_ctx* c = b->ctx;
+    std::vector<uint32_t> cnt_h;
+    const uint32_t* cnt = b->d_tracks;  // = the records counted
+    if (!b->host_res) {
+        cnt_h.resize(b->n_props);
+        PCS_TRY(fetch_results(b, cnt_h.data(), b->d_tracks));
+        PCS_HIP(hipStreamSynchronize(b->stream));
+        cnt = cnt_h.data();
+    }
+    const size_t per = (size_t)c->sys.n_k * c->sys.n_de;
+    const uint32_t chunk =
+        (uint32_t)std::min<size_t>(b->n_props, std::max<size_t>(1, std::min<size_t>(4096, (256u << 20) / (per * 4))));
+    const size_t piece = std::min<size_t>(per * chunk, kHistKeep / 8u);  // words, two of them staged
+    if (per * chunk > b->cap_hist) {
+        b->cap_hist = 0;
+        if (b->h_hist) hipHostFree(b->h_hist);
+        b->h_hist = nullptr;
+        PCS_TRY(dev_alloc(&b->d_hist, per * chunk));
+        const hipError_t e = hipHostMalloc((void**)&b->h_hist, 2u * piece * 4u, hipHostMallocDefault);
+        if (e != hipSuccess) return set_error(PCS_ENOMEM, "hipHostMalloc (histogram staging): %s", hipGetErrorString(e));
+        b->cap_hist = per * chunk;
+    }
+    hipError_t e = hipSuccess;
+    for (uint32_t lo = 0; lo < b->n_props && e == hipSuccess; lo += chunk) {
+        const uint32_t m = std::min(chunk, b->n_props - lo);
+        uint32_t mx = 0;
+        for (uint32_t i = lo; i < lo + m; ++i)  // the kernel caps each count at its slice
+            mx = std::max(mx, b->dev_planned ? cnt[i] : std::min(cnt[i], b->hprops[i].rec_cap));
+        const size_t words = per * m;
+        e = hipMemsetAsync(b->d_hist, 0, words * 4, b->stream);
+        if (e == hipSuccess)
+            e = launch_dense_hist(b->d_props, lo, m, b->d_count, mx, c->sys.n_k, c->sys.n_de, b->d_hist, b->stream);
+        auto fetch = [&](size_t at) -> hipError_t {
+            return hipMemcpyAsync(b->h_hist + (at / piece % 2u) * piece, b->d_hist + at, std::min(piece, words - at) * 4u,
+                                  hipMemcpyDeviceToHost, b->stream);
+        };
+        if (e == hipSuccess) e = fetch(0);
+        for (size_t at = 0; at < words && e == hipSuccess; at += piece) {
+            e = hipStreamSynchronize(b->stream);
+            if (e == hipSuccess && at + piece < words) e = fetch(at + piece);
+            if (e == hipSuccess)
+                std::memcpy(hist_out + per * lo + at, b->h_hist + (at / piece % 2u) * piece, std::min(piece, words - at) * 4u);
+        }
+    }
+    if (b->cap_hist * 4u > kHistKeep) {
+        hipStreamSynchronize(b->stream);
+        hipFree(b->d_hist);
+        hipHostFree(b->h_hist);
+        b->d_hist = b->h_hist = nullptr;
+        b->cap_hist = 0;
+    }
+    if (e != hipSuccess) return hip_error(e, "dense histogram");
+    return PCS_OK;
+}
+
 int pcs_batch_read(pcs_batch* b, double* dist_out, uint32_t* hist_out, uint32_t* tracks_out)
 {
     if (!b) return set_error(PCS_EINVAL, "batch is NULL");
@@ -1015,36 +1156,9 @@ int pcs_batch_read(pcs_batch* b, double* dist_out, uint32_t* hist_out, uint32_t*
     PCS_HIP(hipStreamSynchronize(b->stream));
     PCS_TRY(rerun_overflows(b));
     if (b->n_props == 0) return PCS_OK;
-    if (dist_out)
-        PCS_HIP(hipMemcpyAsync(dist_out, b->d_dist, b->n_props * sizeof(double), hipMemcpyDeviceToHost, b->stream));
-    if (tracks_out)
-        PCS_HIP(hipMemcpyAsync(tracks_out, b->d_tracks, b->n_props * 4, hipMemcpyDeviceToHost, b->stream));
-    if (hist_out) {
-        // Dense histograms are formed from the records in chunks of proposals.
-        std::vector<uint32_t> cnt(b->n_props);
-        PCS_HIP(hipMemcpyAsync(cnt.data(), b->d_count, b->n_props * 4, hipMemcpyDeviceToHost, b->stream));
-        PCS_HIP(hipStreamSynchronize(b->stream));
-        const size_t per = (size_t)c->sys.n_k * c->sys.n_de;
-        const uint32_t chunk = (uint32_t)std::max<size_t>(1, std::min<size_t>(4096, (256u << 20) / (per * 4)));
-        uint32_t* d_h = nullptr;
-        PCS_TRY(dev_alloc(&d_h, per * chunk));
-        int r = PCS_OK;
-        for (uint32_t lo = 0; lo < b->n_props && r == PCS_OK; lo += chunk) {
-            const uint32_t m = std::min(chunk, b->n_props - lo);
-            uint32_t mx = 0;
-            for (uint32_t i = lo; i < lo + m; ++i)  // the kernel caps each count at its slice
-                mx = std::max(mx, b->dev_planned ? cnt[i] : std::min(cnt[i], b->hprops[i].rec_cap));
-            hipError_t e = hipMemsetAsync(d_h, 0, per * m * 4, b->stream);
-            if (e == hipSuccess)
-                e = launch_dense_hist(b->d_props, lo, m, b->d_count, mx, c->sys.n_k, c->sys.n_de, d_h, b->stream);
-            if (e == hipSuccess)
-                e = hipMemcpyAsync(hist_out + per * lo, d_h, per * m * 4, hipMemcpyDeviceToHost, b->stream);
-            if (e == hipSuccess) e = hipStreamSynchronize(b->stream);
-            if (e != hipSuccess) r = hip_error(e, "dense histogram");
-        }
-        hipFree(d_h);
-        PCS_TRY(r);
-    }
+    if (dist_out) PCS_TRY(fetch_results(b, dist_out, b->d_dist));
+    if (tracks_out) PCS_TRY(fetch_results(b, tracks_out, b->d_tracks));
+    if (hist_out) PCS_TRY(read_hist(b, hist_out));
     PCS_HIP(hipStreamSynchronize(b->stream));
     return PCS_OK;
 }
@@ -1106,10 +1220,7 @@ int pcs_batch_propose(pcs_batch* b, const pcs_prior* pr, const double* theta, co
         b->cap_props = 0;
         PCS_TRY(dev_alloc(&b->d_props, n_trials));
         PCS_TRY(dev_alloc(&b->d_count, n_trials));
-        PCS_TRY(dev_alloc(&b->d_tracks, n_trials));
-        PCS_TRY(dev_alloc(&b->d_dist, n_trials));
-        PCS_TRY(dev_alloc(&b->d_exact, n_trials));
-        PCS_TRY(dev_alloc(&b->d_status, n_trials));
+        PCS_TRY(alloc_results(b, n_trials));
         b->cap_props = n_trials;
         relayout = true;
     }
@@ -1350,8 +1461,7 @@ int pcs_batch_read_exact(pcs_batch* b, uint64_t* exact_out)
     if (!b->ran) return set_error(PCS_ESTATE, "batch has not run");
     PCS_HIP(hipSetDevice(b->ctx->device));
     PCS_HIP(hipStreamSynchronize(b->stream));
-    if (b->n_props)
-        PCS_HIP(hipMemcpyAsync(exact_out, b->d_exact, b->n_props * sizeof(uint64_t), hipMemcpyDeviceToHost, b->stream));
+    PCS_TRY(fetch_results(b, exact_out, b->d_exact));
     PCS_HIP(hipStreamSynchronize(b->stream));
     return PCS_OK;
 }
@@ -1788,12 +1898,17 @@ int pcs_simulate(pcs_ctx* c, const pcs_proposal* props, uint32_t n, const uint32
                  uint32_t* hist_out, uint32_t* tracks_out)
 {
     if (!c) return set_error(PCS_EINVAL, "context is NULL");
-    pcs_batch* b = nullptr;
-    PCS_TRY(pcs_batch_create(c, &b));
+    pcs_batch* b = c->oneshot;
+    c->oneshot = nullptr;
+    if (!b) PCS_TRY(pcs_batch_create(c, &b));
     int r = pcs_batch_load(b, props, n, vframes, vparticles, n_videos);
     if (r == PCS_OK) r = pcs_batch_run(b, seed, mode);
     if (r == PCS_OK) r = pcs_batch_read(b, dist_out, hist_out, tracks_out);
-    pcs_batch_destroy(b);
+    if (r == PCS_OK && b->cap_props <= kHostResults && b->cap_arena <= kOneshotKeep && !b->d_rec2) {
+        c->oneshot = b;
+    } else {
+        pcs_batch_destroy(b);
+    }
     return r;
 }
 
