@@ -79,23 +79,25 @@ int validate_proposal(const pcs_system& s, const pcs_proposal& p)
 // Summed-area table of the observed histogram (uint32 like the reference's
 // host SAT, src/gpu/detail/simulation_impl.inl:617-628), in rows of
 // sat_pitch(n_de) with the columns at their right end, its deepest row and
-// its largest entry.
+// a bound of its entries.
 void build_sat(const uint32_t* H, uint32_t n_k, uint32_t n_de, std::vector<uint32_t>& S, uint32_t& maxrow, uint32_t& most)
 {
     const uint32_t pitch = sat_pitch(n_de), pad = pitch - n_de;
     S.assign((size_t)n_k * pitch, 0u);
-    maxrow = most = 0;
+    maxrow = 0;
+    uint64_t all = 0;  // observed tracks: no entry is larger, or wraps, below 2^32 of them
     for (uint32_t i = 0; i < n_k; ++i) {
-        uint32_t run = 0;
+        uint64_t run = 0;
         uint32_t* row = S.data() + (size_t)i * pitch + pad;
         for (uint32_t j = 0; j < n_de; ++j) {
             const uint32_t h = H ? H[(size_t)i * n_de + j] : 0u;
             if (h) maxrow = i;
             run += h;
-            row[j] = run + (i ? row[(ptrdiff_t)j - (ptrdiff_t)pitch] : 0u);
-            most = std::max(most, row[j]);
+            row[j] = (uint32_t)run + (i ? row[(ptrdiff_t)j - (ptrdiff_t)pitch] : 0u);
         }
+        all += run;
     }
+    most = (uint32_t)std::min<uint64_t>(all, 0xffffffffu);
 }
 
 DevSys make_devsys(const pcs_system& s, uint32_t maxrow, uint32_t most, const uint32_t* dsat)
@@ -190,6 +192,8 @@ struct pcs_batch {
     pcs_proposal* d_in = nullptr;
     double *d_theta_pop = nullptr, *d_cumw = nullptr, *d_theta_new = nullptr;
     uint64_t* d_totals = nullptr;  // [0] planned records, [1] tiles
+    uint64_t* d_bsums = nullptr;   // block sums of the device plan
+    size_t cap_bsums = 0;
     size_t cap_in = 0, cap_pop = 0, cap_new = 0;
     uint64_t last_need = 0;      // records the last device plan asked for
     // resident population (pcs_batch_set_population): d_theta_pop, d_cumw
@@ -391,6 +395,7 @@ int device_plan(pcs_batch* b)
     pa.rec_count = b->d_count;
     pa.tile_counter = b->d_tile_counter;
     pa.totals = b->d_totals;
+    pa.block_sums = b->d_bsums;
     PCS_HIP(launch_prepare(pa, b->stream));
     b->planned_ppl = (int)c->tune.particles_per_lane;
     b->host_vtile = false;
@@ -479,8 +484,8 @@ int enqueue_plain(pcs_batch* b, const std::vector<uint32_t>* subset, bool stream
     }
     for (uint32_t i = 0; i < n; ++i) {
         const uint32_t P = subset ? (*subset)[i] : i;
-        const pcs_proposal& p = b->props[P];
-        const uint32_t lo = b->vtile[p.first_video], hi = b->vtile[p.first_video + p.n_videos];
+        const uint32_t v0 = b->dev_planned ? P * b->J : b->props[P].first_video;
+        const uint32_t lo = b->vtile[v0], hi = b->vtile[v0 + (b->dev_planned ? b->J : b->props[P].n_videos)];
         hipStream_t s = streams ? b->pstream[i % PCS_PLAIN_STREAMS] : b->stream;
         PCS_HIP(launch_walk(walk_args(b, lo, hi), (int)t.particles_per_lane, (int)t.waves_per_group, false, 0, gauss,
                             zref, s));
@@ -865,7 +870,7 @@ int pcs_batch_destroy(pcs_batch* b)
     destroy_graph(b);
     void* ptrs[] = {b->d_props, b->d_vframes, b->d_vparticles, b->d_vprop, b->d_vtile, b->d_rec, b->d_srt,
                     b->d_rec2, b->d_srt2, b->d_count, b->d_tile_counter, b->d_hist,
-                    b->d_seed, b->d_in, b->d_theta_pop, b->d_cumw, b->d_theta_new, b->d_totals, b->d_wpop,
+                    b->d_seed, b->d_in, b->d_theta_pop, b->d_cumw, b->d_theta_new, b->d_totals, b->d_bsums, b->d_wpop,
                     b->d_xn, b->d_xo, b->d_wsum, b->d_part, b->d_dscratch};
     for (void* p : ptrs)
         if (p) hipFree(p);
@@ -1249,19 +1254,19 @@ int pcs_batch_propose(pcs_batch* b, const pcs_prior* pr, const double* theta, co
     }
     b->new_P = P;
     if (!b->d_totals) PCS_TRY(dev_alloc(&b->d_totals, 2));
+    const size_t nb = (size_t)plan_blocks(n_trials) + plan_blocks(nv);
+    if (nb > b->cap_bsums) {
+        b->cap_bsums = 0;
+        PCS_TRY(dev_alloc(&b->d_bsums, nb));
+        b->cap_bsums = nb;
+    }
     b->dev_planned = true;
     b->host_vtile = false;
     b->J = J;
     b->n_props = n_trials;
     b->n_videos = nv;
     b->ran = false;
-    // host side of the plan: proposal i owns videos [i J, (i + 1) J)
-    b->props.assign(n_trials, pcs_proposal{});
-    for (uint32_t i = 0; i < n_trials; ++i) {
-        b->props[i].sim_id = first_sim_id + i;
-        b->props[i].first_video = i * J;
-        b->props[i].n_videos = J;
-    }
+    b->props.clear();  // proposal i owns videos [i J, (i + 1) J)
     b->hprops.clear();
     b->vframes.clear();
     b->vparticles.clear();

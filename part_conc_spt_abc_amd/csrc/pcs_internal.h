@@ -30,7 +30,7 @@ struct DevSys {
     uint32_t dist_kind;
     uint32_t maxrow_obs;      // last row holding observed tracks (0 if none)
     const uint32_t* obs_sat;  // observed summed-area table, n_k rows of sat_pitch(n_de) uint32
-    uint32_t obs_max;         // its largest entry
+    uint32_t obs_max;         // bound of its entries
     uint32_t pad1;
 };
 static_assert(sizeof(DevSys) == 80, "DevSys layout");
@@ -235,7 +235,7 @@ struct LoopArgs {
 };
 
 // Tables of a batch built on the device from the caller's proposal records
-// (prepare_kernel): per proposal its DevProp with a record slice placed in
+// (launch_prepare): per proposal its DevProp with a record slice placed in
 // [rec, rec + arena_cap) (slices past the arena's end are cut short and
 // overflow), per video its proposal and tile prefix. Proposals hold
 // consecutive video ranges: props[i].first_video = sum of earlier n_videos.
@@ -257,7 +257,9 @@ struct PrepArgs {
     uint32_t* rec_count;      // zeroed
     uint32_t* tile_counter;   // zeroed
     uint64_t* totals;         // [0] planned records, [1] tiles
+    uint64_t* block_sums;     // plan_blocks(n) + plan_blocks(n_videos) entries; nullable: one workgroup plans all
 };
+inline uint32_t plan_blocks(uint32_t n) { return (uint32_t)(((uint64_t)n + 1023u) / 1024u); }
 
 // Proposal step of an ABC-PMC round (propose_kernel), one wave per trial:
 // parent by cumulative weight, displaced parameters reflected into the prior,

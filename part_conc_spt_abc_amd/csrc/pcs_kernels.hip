@@ -1150,10 +1150,8 @@ __global__ __launch_bounds__(kGrpThreads) void walk_group_kernel(WalkArgs a)
                         de_first = (__float_as_uint(q.de) & at) | (de_first & ~at);
                         q.de = __uint_as_float(__float_as_uint(q.de + step2) & keep);
                     };
-                    // Two chunks a turn, the path without other closes laid
-                    // out straight: a lone wave loses 40 cycles or more to a
-                    // branch it takes.
-#pragma unroll 2
+                    // The path without other closes is laid out straight: a
+                    // lone wave loses 40 cycles or more to a branch it takes.
                     for (uint32_t j = 0; 4u * j < n; ++j) {
                         const f32x4 r1 = rs[min(j + 1u, (uint32_t)kGrpProd - 1u) * kWave];
                         if (__builtin_expect(4u * j + 4u > n, 0)) {  // frames past the last add nothing
@@ -2747,58 +2745,70 @@ __device__ uint64_t block_scan_u64(uint64_t v, uint64_t* sh, uint64_t& total)
     return base + x - v;
 }
 
-// Device-side plan of a batch (one workgroup): record slices by the
-// capacity estimate, prefix-summed into the arena; video -> proposal map;
-// tile prefix. Proposals (videos) go in rounds of 1024, thread t taking
-// element r * 1024 + t, so that each round's loads and stores are coalesced.
+// Device-side plan of a batch: record slices by the capacity estimate,
+// prefix-summed into the arena; video -> proposal map; tile prefix. Both sums
+// run over blocks of 1,024 proposals (videos), thread t taking element t of its
+// block, so that loads and stores are coalesced.
+__device__ __forceinline__ uint64_t plan_records(const PrepArgs& a, uint32_t i)
+{
+    if (i >= a.n) return 0ull;
+    const pcs_proposal& p = a.in[i];
+    return slice_capacity(a.sys[0], p.half_az, p.n_videos, a.vframes + p.first_video, a.vparticles + p.first_video,
+                          a.cap_factor);
+}
+
+__device__ __forceinline__ uint64_t plan_tiles(const PrepArgs& a, uint32_t v)
+{
+    return v < a.n_videos ? (a.vparticles[v] + a.tile_particles - 1u) / a.tile_particles : 0ull;
+}
+
+// Proposal i, its slice at record `off` of the plan.
+__device__ __forceinline__ void plan_proposal(const PrepArgs& a, uint32_t i, uint64_t cap, uint64_t off)
+{
+    if (i >= a.n) return;
+    const pcs_proposal& p = a.in[i];
+    const uint64_t at = off < a.arena_cap ? off : a.arena_cap;
+    const uint64_t room = a.arena_cap - at;
+    DevProp d;
+    d.sim_id = p.sim_id;
+    d.first_video = p.first_video;
+    d.n_videos = p.n_videos;
+    d.sys_id = 0u;
+    d.rec = a.rec + at;
+    d.srt = a.srt + at;
+    d.rec_cap = (uint32_t)(cap < room ? cap : room);
+    d.key0 = 0u;
+    d.key1 = 0u;
+    d.pad = 0u;
+    for (int c = 0; c < PCS_MAX_SPECIES; ++c) {
+        d.half_az[c] = p.half_az[c];
+        d.cum_prob[c] = p.cum_prob[c];
+        d.sigma[c] = p.sigma[c];
+    }
+    a.props[i] = d;
+    a.rec_count[i] = 0u;
+    for (uint32_t v = p.first_video; v < p.first_video + p.n_videos; ++v) a.vprop[v] = i;
+}
+
+// The whole plan in one workgroup, block after block: for batches of a few
+// blocks, where the launches below would cost more.
 __global__ __launch_bounds__(kPrepThreads) void prepare_kernel(PrepArgs a)
 {
     __shared__ uint64_t sh[2 * kPrepWaves];
     const uint32_t tid = threadIdx.x;
-    const DevSys& sy = a.sys[0];
     uint64_t base = 0ull;
     for (uint32_t r0 = 0; r0 < a.n; r0 += kPrepThreads) {
-        const uint32_t i = r0 + tid;
-        uint64_t cap = 0ull;
-        if (i < a.n) {
-            const pcs_proposal& p = a.in[i];
-            cap = slice_capacity(sy, p.half_az, p.n_videos, a.vframes + p.first_video, a.vparticles + p.first_video,
-                                 a.cap_factor);
-        }
+        const uint64_t cap = plan_records(a, r0 + tid);
         uint64_t round_total;
         const uint64_t off = base + block_scan_u64(cap, sh, round_total);
-        if (i < a.n) {
-            const pcs_proposal& p = a.in[i];
-            const uint64_t at = off < a.arena_cap ? off : a.arena_cap;
-            const uint64_t room = a.arena_cap - at;
-            DevProp d;
-            d.sim_id = p.sim_id;
-            d.first_video = p.first_video;
-            d.n_videos = p.n_videos;
-            d.sys_id = 0u;
-            d.rec = a.rec + at;
-            d.srt = a.srt + at;
-            d.rec_cap = (uint32_t)(cap < room ? cap : room);
-            d.key0 = 0u;
-            d.key1 = 0u;
-            d.pad = 0u;
-            for (int c = 0; c < PCS_MAX_SPECIES; ++c) {
-                d.half_az[c] = p.half_az[c];
-                d.cum_prob[c] = p.cum_prob[c];
-                d.sigma[c] = p.sigma[c];
-            }
-            a.props[i] = d;
-            a.rec_count[i] = 0u;
-            for (uint32_t v = p.first_video; v < p.first_video + p.n_videos; ++v) a.vprop[v] = i;
-        }
+        plan_proposal(a, r0 + tid, cap, off);
         base += round_total;
     }
     uint64_t tbase = 0ull;
     for (uint32_t r0 = 0; r0 < a.n_videos; r0 += kPrepThreads) {
         const uint32_t v = r0 + tid;
-        const uint64_t tiles = v < a.n_videos ? (a.vparticles[v] + a.tile_particles - 1u) / a.tile_particles : 0ull;
         uint64_t round_total;
-        const uint64_t t = tbase + block_scan_u64(tiles, sh, round_total);
+        const uint64_t t = tbase + block_scan_u64(plan_tiles(a, v), sh, round_total);
         if (v < a.n_videos) a.vtile[v] = (uint32_t)t;
         tbase += round_total;
     }
@@ -2807,6 +2817,62 @@ __global__ __launch_bounds__(kPrepThreads) void prepare_kernel(PrepArgs a)
         a.totals[0] = base;
         a.totals[1] = tbase;
         *a.tile_counter = 0u;
+    }
+}
+
+// The plan over many workgroups, one per block of proposals, then one per block
+// of videos: the blocks' sums, their scan, and the tables. (One workgroup's
+// memory path bound the single kernel: 1.31 ms for 100,000 trials, 166 us for
+// 2,000 of 25 videos.)
+__global__ __launch_bounds__(kPrepThreads) void plan_sums_kernel(PrepArgs a, uint32_t prop_blocks)
+{
+    __shared__ uint64_t sh[2 * kPrepWaves];
+    const uint32_t b = blockIdx.x;
+    const uint64_t x = b < prop_blocks ? plan_records(a, b * kPrepThreads + threadIdx.x)
+                                       : plan_tiles(a, (b - prop_blocks) * kPrepThreads + threadIdx.x);
+    uint64_t total;
+    block_scan_u64(x, sh, total);
+    if (threadIdx.x == 0) a.block_sums[b] = total;
+}
+
+__global__ __launch_bounds__(kPrepThreads) void plan_scan_kernel(PrepArgs a, uint32_t prop_blocks, uint32_t video_blocks)
+{
+    __shared__ uint64_t sh[2 * kPrepWaves];
+    const uint32_t tid = threadIdx.x;
+    for (uint32_t part = 0; part < 2u; ++part) {
+        uint64_t* s = a.block_sums + (part ? prop_blocks : 0u);
+        const uint32_t n = part ? video_blocks : prop_blocks;
+        uint64_t base = 0ull;
+        for (uint32_t r0 = 0; r0 < n; r0 += kPrepThreads) {
+            const uint32_t i = r0 + tid;
+            const uint64_t x = i < n ? s[i] : 0ull;
+            uint64_t total;
+            const uint64_t ex = base + block_scan_u64(x, sh, total);
+            if (i < n) s[i] = ex;
+            base += total;
+        }
+        if (tid == 0) {
+            a.totals[part] = base;
+            if (part) a.vtile[a.n_videos] = (uint32_t)base;
+        }
+    }
+    if (tid == 0) *a.tile_counter = 0u;
+}
+
+__global__ __launch_bounds__(kPrepThreads) void plan_write_kernel(PrepArgs a, uint32_t prop_blocks)
+{
+    __shared__ uint64_t sh[2 * kPrepWaves];
+    const uint32_t b = blockIdx.x;
+    uint64_t total;
+    if (b < prop_blocks) {
+        const uint32_t i = b * kPrepThreads + threadIdx.x;
+        const uint64_t cap = plan_records(a, i);
+        const uint64_t off = a.block_sums[b] + block_scan_u64(cap, sh, total);
+        plan_proposal(a, i, cap, off);
+    } else {
+        const uint32_t v = (b - prop_blocks) * kPrepThreads + threadIdx.x;
+        const uint64_t t = a.block_sums[b] + block_scan_u64(plan_tiles(a, v), sh, total);
+        if (v < a.n_videos) a.vtile[v] = (uint32_t)t;
     }
 }
 
@@ -3123,36 +3189,55 @@ __global__ __launch_bounds__(256) void pmc_sums_kernel(const double* xn, uint32_
 }
 
 // Cumulative weights in member order: the same FP64 sums as a sequential
-// cumsum. One wave loads kCumLoads x 64 weights at a time (coalesced, all in
-// flight), then one running sum passes through them lane by lane (readlane of
-// each weight, a wave-uniform add), and each lane keeps the sum at its member.
-constexpr int kCumLoads = 8;
-__global__ __launch_bounds__(kWave) void cumsum_kernel(const double* w, uint32_t n, double* cum)
+// cumsum. The sum itself is one chain of dependent additions, so all else is
+// kept off it: in round i waves 1..3 load tile i into LDS and store tile
+// i - 2's sums, while lane 0 adds through tile i - 1 in place, 16 weights read
+// ahead of the 16 being added. Bound by the additions' latency. (Each weight
+// broadcast by readlane between the additions, 100,000 members took 4.4 ms.)
+constexpr uint32_t kCumTile = 2048;
+__global__ __launch_bounds__(256) void cumsum_kernel(const double* w, uint32_t n, double* cum)
 {
-    const uint32_t lane = threadIdx.x;
+    typedef double f64x2 __attribute__((ext_vector_type(2)));
+    __shared__ __align__(16) double buf[3][kCumTile];
+    const uint32_t tid = threadIdx.x;
+    const uint32_t nt = (n + kCumTile - 1u) / kCumTile;
     double acc = 0.0;
-    for (uint32_t base = 0; base < n; base += (uint32_t)(kCumLoads * kWave)) {
-        double v[kCumLoads];
-#pragma unroll
-        for (int u = 0; u < kCumLoads; ++u) {
-            const uint32_t i = base + (uint32_t)u * kWave + lane;
-            v[u] = i < n ? w[i] : 0.0;
-        }
-#pragma unroll
-        for (int u = 0; u < kCumLoads; ++u) {
-            const uint32_t first = base + (uint32_t)u * kWave;
-            if (first >= n) break;
-            const uint32_t nl = min((uint32_t)kWave, n - first);
-            const uint64_t bits = __double_as_longlong(v[u]);
-            double mine = 0.0;
-            for (uint32_t l = 0; l < nl; ++l) {
-                const uint32_t lo = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)bits, (int)l);
-                const uint32_t hi = (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(bits >> 32), (int)l);
-                acc += __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
-                mine = (lane == l) ? acc : mine;
+    for (uint32_t it = 0; it < nt + 2u; ++it) {
+        if (tid >= (uint32_t)kWave) {
+            for (uint32_t j = tid - kWave; j < kCumTile; j += 256u - kWave) {
+                if (it >= 2u) {
+                    const uint32_t i = (it - 2u) * kCumTile + j;
+                    if (i < n) cum[i] = buf[(it - 2u) % 3u][j];
+                }
+                if (it < nt) {
+                    const uint32_t i = it * kCumTile + j;
+                    buf[it % 3u][j] = i < n ? w[i] : 0.0;
+                }
             }
-            if (lane < nl) cum[first + lane] = mine;
+        } else if (tid == 0u && it >= 1u && it <= nt) {
+            f64x2* p = reinterpret_cast<f64x2*>(buf[(it - 1u) % 3u]);
+            f64x2 a[8], b[8];
+#pragma unroll
+            for (int q = 0; q < 8; ++q) a[q] = p[q];
+            for (uint32_t j = 0; j < kCumTile / 2u; j += 8u) {
+                const uint32_t nx = min(j + 8u, kCumTile / 2u - 8u);
+#pragma unroll
+                for (int q = 0; q < 8; ++q) b[q] = p[nx + q];
+#pragma unroll
+                for (int q = 0; q < 8; ++q) {
+                    acc += a[q].x;
+                    a[q].x = acc;
+                    acc += a[q].y;
+                    a[q].y = acc;
+                }
+#pragma unroll
+                for (int q = 0; q < 8; ++q) {
+                    p[j + q] = a[q];
+                    a[q] = b[q];
+                }
+            }
         }
+        __syncthreads();
     }
 }
 
@@ -3510,7 +3595,14 @@ hipError_t launch_serve_loop(const LoopArgs& a, uint32_t grid, uint32_t n_de_max
 hipError_t launch_prepare(const PrepArgs& a, hipStream_t s)
 {
     (void)hipGetLastError();  // report only this launch's error
-    hipLaunchKernelGGL(prepare_kernel, dim3(1), dim3(kPrepThreads), 0, s, a);
+    const uint32_t pb = plan_blocks(a.n), vb = plan_blocks(a.n_videos);
+    if (!a.block_sums || pb + vb <= 4u) {  // 3 launches of 3 us against 4 us a block
+        hipLaunchKernelGGL(prepare_kernel, dim3(1), dim3(kPrepThreads), 0, s, a);
+        return hipGetLastError();
+    }
+    hipLaunchKernelGGL(plan_sums_kernel, dim3(pb + vb), dim3(kPrepThreads), 0, s, a, pb);
+    hipLaunchKernelGGL(plan_scan_kernel, dim3(1), dim3(kPrepThreads), 0, s, a, pb, vb);
+    hipLaunchKernelGGL(plan_write_kernel, dim3(pb + vb), dim3(kPrepThreads), 0, s, a, pb);
     return hipGetLastError();
 }
 
@@ -3526,7 +3618,7 @@ hipError_t launch_cumsum(const double* w, uint32_t n, double* cum, hipStream_t s
 {
     (void)hipGetLastError();  // report only this launch's error
     if (n == 0) return hipSuccess;
-    hipLaunchKernelGGL(cumsum_kernel, dim3(1), dim3(kWave), 0, s, w, n, cum);
+    hipLaunchKernelGGL(cumsum_kernel, dim3(1), dim3(256), 0, s, w, n, cum);
     return hipGetLastError();
 }
 
