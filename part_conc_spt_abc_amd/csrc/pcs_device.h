@@ -133,15 +133,19 @@ constexpr float kLogTiny = 0x1p-100f;
 // between two floats (rounded up instead of to even).
 __device__ __forceinline__ float neg2log_u24(uint32_t w)
 {
-    // x = m 2^e with m in [sqrt(1/2), sqrt(2)), in integer steps on the bits
-    // of x: t = bits(x) - bits(sqrt(1/2)) - (32 << 23) carries e - 32 in its
-    // top 9 bits (arithmetic shift) and m's bits are the low 23 bits of t plus
-    // bits(sqrt(1/2)) (a borrow from the mantissa lands m in [1, sqrt 2)).
-    // Same m and e as frexp followed by the sqrt(1/2) fold-up.
-    const int32_t t = (int32_t)(__float_as_uint((float)(w | 0xffu)) - (kSqrtHalfBits + (32u << 23)));
-    const float m = __uint_as_float(((uint32_t)t & 0x7fffffu) + kSqrtHalfBits);
-    const float g = __builtin_fmaf(m, -2.0f, 2.0f);  // exact (Sterbenz)
-    const float E = (float)(t >> 23);
+    // x = m 2^32 2^E with m in [sqrt(1/2), sqrt(2)), in integer steps on the
+    // bits of x: bits(x) - bits(sqrt(1/2)) - (32 << 23) carries E in its top 9
+    // bits, hi = E 2^23 as an integer, and taking hi off the exponent of x
+    // leaves m 2^32 (a borrow from the mantissa lands m in [1, sqrt 2)). Same m
+    // and E as frexp followed by the sqrt(1/2) fold-up; E 2^23 and m 2^32 enter
+    // the multiply-adds with their powers of two taken into the constants. (An
+    // instruction less a logarithm than E and m themselves: the walk of 4,000
+    // mixed simulations 15.84 -> 15.58 ms.)
+    const uint32_t xb = __float_as_uint((float)(w | 0xffu));
+    const int32_t hi = (int32_t)(xb - (kSqrtHalfBits + (32u << 23))) & (int32_t)0xff800000;
+    const float m32 = __uint_as_float(xb - (uint32_t)hi);
+    const float g = __builtin_fmaf(m32, -0x1p-31f, 2.0f);  // exact (Sterbenz)
+    const float E23 = (float)hi;
     const float g2 = __builtin_fmaf(g, g, kLogTiny);
     float Q = kLogQ6;
     Q = __builtin_fmaf(Q, g, kLogQ5);
@@ -150,7 +154,7 @@ __device__ __forceinline__ float neg2log_u24(uint32_t w)
     Q = __builtin_fmaf(Q, g, kLogQ2);
     Q = __builtin_fmaf(Q, g, kLogQ1);
     Q = __builtin_fmaf(Q, g, kLogQ0);
-    return __builtin_fmaf(E, kNeg2Ln2, __builtin_fmaf(g2, Q, g));
+    return __builtin_fmaf(E23, kNeg2Ln2 * 0x1p-23f, __builtin_fmaf(g2, Q, g));
 }
 
 // 2^f = 1 + f Q(f) on [0, 1); Q from fit_math_coeffs.py (within 1.07 ulp of 2^f,
