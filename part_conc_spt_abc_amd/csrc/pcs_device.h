@@ -189,6 +189,23 @@ __device__ __forceinline__ bool gauss_detect(float z, float c, uint32_t w)
     return (float)(w | 0xffu) <= t;
 }
 
+// The same test from the hardware's 2^v (within 1 ulp, so within 2^-21 of the
+// polynomial's): decided unless x lies within 2^-20 of the bound, where some
+// lane then takes the exact form above (once in 10^4 wave-steps). A bound
+// below the normal floats or a NaN detects nothing in either form. For whole
+// waves of a full GPU, where instructions count (24 large simulations: walk
+// 4.34 -> 4.25 ms); a lone wave's chain is longer by the branch (152 tiles
+// walked by groups: 127 -> 149 us), so the group walks keep the exact form.
+__device__ __forceinline__ bool gauss_test(float z, float c, uint32_t w)
+{
+    const float t = __builtin_amdgcn_exp2f(__builtin_fmaf(-c, z * z, 32.0f));
+    const float d = (float)(w | 0xffu) - t;
+    bool in = d <= 0.0f;
+    if (__builtin_expect(__builtin_amdgcn_ballot_w64(__builtin_fabsf(d) <= t * 0x1p-20f) != 0ull, 0))
+        in = gauss_detect(z, c, w);
+    return in;
+}
+
 // Correctly rounded sqrt for the Box-Muller radius y = -2 ln u (2^-100 Q(0) =
 // 0x1.00006p-102 at u = 1, else 1.19e-7 <= y <= 33.3): s = y rsq(y) with one
 // correction by the residual y - s^2 (Markstein). It equals the correctly

@@ -483,7 +483,7 @@ __device__ __forceinline__ void step_particle(Particle& q, uint64_t m_active, ui
         q.z = wrap_reflect(zn, K.hz);
     }
     const bool cx = q.x <= K.wx, cy = q.y <= K.wy;
-    const bool cz = GAUSS ? gauss_detect(ZBOX ? q.z - 0.5f : q.z, K.cg, wdet)
+    const bool cz = GAUSS ? gauss_test(ZBOX ? q.z - 0.5f : q.z, K.cg, wdet)
                           : (ZBOX ? q.z <= q.wz : __builtin_fabsf(q.z) <= q.wz);
     // Lanes inside the window and lanes closing a track: wave masks formed
     // from the masks of the single comparisons (no per-lane boolean is
