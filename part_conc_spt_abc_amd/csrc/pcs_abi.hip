@@ -6,6 +6,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <functional>
 #include <mutex>
 #include <new>
 #include <string>
@@ -159,6 +160,11 @@ struct pcs_batch {
     std::vector<uint32_t> vframes, vparticles, vprop, vtile;
     uint32_t n_props = 0, n_videos = 0, n_tiles = 0;
     int planned_ppl = 0;
+    // tiles of the batched form taken longest video first (plan_tiles)
+    bool ordered = false;
+    std::vector<uint32_t> vorder, otile;
+    uint32_t *d_vorder = nullptr, *d_otile = nullptr;
+    size_t cap_order = 0;
     uint64_t arena_records = 0;
     uint32_t* d_rec2 = nullptr;  // rerun arena of the last run (overflowed slices)
     uint32_t* d_srt2 = nullptr;
@@ -331,7 +337,15 @@ int check_tuning(const pcs_tuning& t)
     return PCS_OK;
 }
 
-// Tiles of 64*ppl particles per video, prefix-summed.
+// Tiles beyond which the order of the videos no longer matters: 16 rounds of
+// the GPU's 8,192 wave slots. Up to two tiles a CU all of them start at once.
+constexpr uint32_t kOrderTiles = 16u * 8192u;
+
+// Tiles of 64*ppl particles per video, prefix-summed. Videos of different
+// lengths: the batched form takes them longest first, so that what is still
+// running when the tiles run out is short (500 simulations of 500 to 2,000
+// frames, 21,842 tiles: walk 2.77 -> 2.45 ms; 1,501 of 101 to 999, 11,530
+// tiles: 0.90 -> 0.73 ms; 16 rounds of tiles: 2 % at most).
 void plan_tiles(pcs_batch* b, int ppl)
 {
     const uint32_t tp = 64u * (uint32_t)ppl;
@@ -344,10 +358,35 @@ void plan_tiles(pcs_batch* b, int ppl)
     b->vtile[b->n_videos] = acc;
     b->n_tiles = acc;
     b->planned_ppl = ppl;
+    const auto& f = b->vframes;
+    b->ordered = acc > 2u * (uint32_t)b->ctx->n_cu && acc <= kOrderTiles &&
+                 std::adjacent_find(f.begin(), f.end(), std::not_equal_to<uint32_t>()) != f.end();
+    if (!b->ordered) return;
+    b->vorder.resize(b->n_videos);
+    for (uint32_t v = 0; v < b->n_videos; ++v) b->vorder[v] = v;
+    std::stable_sort(b->vorder.begin(), b->vorder.end(), [&f](uint32_t x, uint32_t y) { return f[x] > f[y]; });
+    b->otile.resize(b->n_videos + 1);
+    acc = 0;
+    for (uint32_t i = 0; i < b->n_videos; ++i) {
+        b->otile[i] = acc;
+        acc += (b->vparticles[b->vorder[i]] + tp - 1u) / tp;
+    }
+    b->otile[b->n_videos] = acc;
 }
 
 int upload_plan(pcs_batch* b)
 {
+    if (b->ordered) {
+        const size_t n = b->otile.size();
+        if (n > b->cap_order) {
+            b->cap_order = 0;
+            PCS_TRY(dev_alloc(&b->d_vorder, n));
+            PCS_TRY(dev_alloc(&b->d_otile, n));
+            b->cap_order = n;
+        }
+        PCS_HIP(hipMemcpyAsync(b->d_vorder, b->vorder.data(), (n - 1u) * 4u, hipMemcpyHostToDevice, b->stream));
+        PCS_HIP(hipMemcpyAsync(b->d_otile, b->otile.data(), n * 4u, hipMemcpyHostToDevice, b->stream));
+    }
     PCS_HIP(hipMemcpyAsync(b->d_vtile, b->vtile.data(), b->vtile.size() * 4, hipMemcpyHostToDevice, b->stream));
     return PCS_OK;
 }
@@ -443,8 +482,12 @@ int enqueue_batched(pcs_batch* b, bool with_events)
     PCS_HIP(launch_reset(b->d_count, b->n_props, b->d_tile_counter, b->stream));
     if (with_events) PCS_HIP(hipEventRecord(b->ev[1], b->stream));
     const uint32_t grid = (uint32_t)c->n_cu * t.groups_per_cu;
-    PCS_HIP(launch_walk(walk_args(b, 0, b->dev_planned ? 0xffffffffu : b->n_tiles), (int)t.particles_per_lane,
-                        (int)t.waves_per_group, true, grid, gauss, zref, b->stream));
+    WalkArgs wa = walk_args(b, 0, b->dev_planned ? 0xffffffffu : b->n_tiles);
+    if (b->ordered && !b->dev_planned) {
+        wa.vtile = b->d_otile;
+        wa.vorder = b->d_vorder;
+    }
+    PCS_HIP(launch_walk(wa, (int)t.particles_per_lane, (int)t.waves_per_group, true, grid, gauss, zref, b->stream));
     if (with_events) PCS_HIP(hipEventRecord(b->ev[2], b->stream));
     PCS_HIP(launch_distance(dist_args(b, 0, b->n_props), c->sys.n_k, c->sys.n_de, b->stream));
     if (with_events) PCS_HIP(hipEventRecord(b->ev[3], b->stream));
@@ -869,7 +912,7 @@ int pcs_batch_destroy(pcs_batch* b)
     if (b->wstream) hipStreamSynchronize(b->wstream);
     destroy_graph(b);
     void* ptrs[] = {b->d_props, b->d_vframes, b->d_vparticles, b->d_vprop, b->d_vtile, b->d_rec, b->d_srt,
-                    b->d_rec2, b->d_srt2, b->d_count, b->d_tile_counter, b->d_hist,
+                    b->d_rec2, b->d_srt2, b->d_count, b->d_tile_counter, b->d_hist, b->d_vorder, b->d_otile,
                     b->d_seed, b->d_in, b->d_theta_pop, b->d_cumw, b->d_theta_new, b->d_totals, b->d_bsums, b->d_wpop,
                     b->d_xn, b->d_xo, b->d_wsum, b->d_part, b->d_dscratch};
     for (void* p : ptrs)

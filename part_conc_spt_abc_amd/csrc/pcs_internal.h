@@ -98,6 +98,7 @@ struct WalkArgs {
     const uint32_t* vparticles;
     const uint32_t* vprop;
     const uint32_t* vtile;   // n_videos + 1 entries
+    const uint32_t* vorder;  // nullable: the videos in the order that vtile takes them in
     uint32_t n_videos;
     uint32_t tile_lo, tile_hi;  // tiles processed by this launch
     uint32_t stage_cap;         // LDS records per wave

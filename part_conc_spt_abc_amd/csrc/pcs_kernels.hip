@@ -797,30 +797,32 @@ __device__ __forceinline__ void walk_tile_coop(const DevProp& pr, const DevSys& 
     }
 }
 
-// Tile t of a batch plan: the video owning it is the largest v with
-// vtile[v] <= t (wave-uniform binary search).
-__device__ __forceinline__ uint32_t tile_video(const WalkArgs& a, uint32_t t)
+// Tile t of a batch plan: the video owning it is the one at the largest place
+// with vtile[place] <= t (wave-uniform binary search); first: its first tile.
+__device__ __forceinline__ uint32_t tile_video(const WalkArgs& a, uint32_t t, uint32_t& first)
 {
     uint32_t lo = 0u, hi = a.n_videos;
     while (hi - lo > 1u) {
         const uint32_t mid = (lo + hi) >> 1;
         if (a.vtile[mid] <= t) lo = mid; else hi = mid;
     }
-    return lo;
+    first = a.vtile[lo];
+    return a.vorder ? a.vorder[lo] : lo;
 }
 
 template <int PPL, bool GAUSS, bool ZREF, bool TRACKS>
 __device__ __forceinline__ void process_tile(const WalkArgs& a, uint32_t t, Stage& st, const float2* tab,
                                              uint32_t s0, uint32_t s1)
 {
-    const uint32_t v = tile_video(a, t);
+    uint32_t first;
+    const uint32_t v = tile_video(a, t, first);
     const uint32_t P = a.vprop[v];
     const DevProp& pr = a.props[P];
     st.rec = pr.rec;
     st.slice_cap = pr.rec_cap;
     st.counter = a.rec_count + P;
     walk_tile<PPL, GAUSS, ZREF, TRACKS>(pr, a.sys[pr.sys_id], a.vframes[v], a.vparticles[v], v - pr.first_video,
-                                        (t - a.vtile[v]) * (uint32_t)(kWave * PPL), st, tab, s0, s1);
+                                        (t - first) * (uint32_t)(kWave * PPL), st, tab, s0, s1);
 }
 
 template <int PPL, bool PERSIST, bool GAUSS, bool ZREF, bool TRACKS = false>
@@ -967,14 +969,15 @@ __global__ __launch_bounds__(kGrpThreads) void walk_group_kernel(WalkArgs a)
     const uint32_t wave = uniform(threadIdx.x / kWave), lane = lane_id();
 
     for (uint32_t t = a.tile_lo + blockIdx.x; t < a.tile_hi; t += gridDim.x) {
-        const uint32_t v = uniform(tile_video(a, t));
+        uint32_t first;
+        const uint32_t v = uniform(tile_video(a, t, first));
         const uint32_t P = uniform(a.vprop[v]);
         const DevProp& pr = a.props[P];
         const DevSys& sy = a.sys[pr.sys_id];
         const uint32_t N = uniform(a.vparticles[v]), F = uniform(a.vframes[v]);
         const uint32_t video = uniform(v - pr.first_video), sim = uniform(pr.sim_id);
         const uint32_t k0 = uniform((uint32_t)seed ^ pr.key0), k1 = uniform((uint32_t)(seed >> 32) ^ pr.key1);
-        const uint32_t id = (t - uniform(a.vtile[v])) * (uint32_t)kWave + lane;
+        const uint32_t id = (t - uniform(first)) * (uint32_t)kWave + lane;
         const WalkConsts K = walk_consts<GAUSS, ZREF>(sy);
         const uint32_t steps = F > 0u ? F - 1u : 0u;
         const uint32_t nr = (steps + kGrpSteps - 1u) / kGrpSteps;

@@ -99,3 +99,26 @@ def test_histograms_through_staging(gpu_lib, n_k, n_de, n):
                 _, t, h = simulate(c2, [p], f[i:i + 1], parts[i:i + 1], 5, 0, True)
                 assert t[0] == tracks[i] and np.array_equal(h[0], H[i])
         b.close()
+
+
+@pytest.mark.parametrize("ppl", [1, 2])
+def test_longest_videos_first(gpu_lib, ppl):
+    """Videos of different lengths are taken longest first in the batched form;
+    each simulation's result is its own (plain form, videos as given)."""
+    model = cases.headline_model(n_k=100, n_de=64)
+    rng = np.random.default_rng(4)
+    props, f, parts = cases.draw_proposals(model, 90, rng, frames_choices=(2, 17, 40, 41, 77), videos=3,
+                                           c_range=(5e6, 3e9))
+    parts[4] = parts[100] = 0
+    with Context(model) as ctx:
+        ctx.set_tuning(particles_per_lane=ppl)
+        b = ctx.batch()
+        for frames in (f, np.full_like(f, 50), f[::-1].copy()):
+            b.load(props, frames, parts)
+            got = []
+            for mode in (1, 1, 0, 3, 2):
+                b.run(3, mode)
+                _, tracks, _ = b.read()
+                got.append((tracks, b.read_exact()))
+            assert all(np.array_equal(x, got[0][0]) and np.array_equal(y, got[0][1]) for x, y in got[1:])
+        b.close()
