@@ -1442,7 +1442,7 @@ int pcs_batch_pmc_weights_async(pcs_batch* b, const double* tau)
     PCS_TRY(grow(&b->d_xn, b->cap_xn, (size_t)sr.n_rows * n_new));
     PCS_TRY(grow(&b->d_xo, b->cap_xo, (size_t)sr.n_rows * n_old));
     PCS_TRY(grow(&b->d_wsum, b->cap_wsum, n_new));
-    PCS_TRY(grow(&b->d_part, b->cap_part, (size_t)pmc_chunks(n_old) * n_new));
+    PCS_TRY(grow(&b->d_part, b->cap_part, (size_t)pmc_chunks(n_new, n_old) * n_new));
     // after the proposal step (recorded by pcs_batch_propose), not after
     // whatever the batch stream has taken since: a walk enqueued before this
     // call runs beside the weights
@@ -1773,7 +1773,7 @@ int pcs_pmc_weights(int device, const double* theta_new, uint32_t n_new, const d
     grow(&wk.xo, wk.cap[1], xo.size() + 1);
     grow(&wk.w, wk.cap[2], (size_t)n_old + 1);
     grow(&wk.s, wk.cap[3], n_new);
-    grow(&wk.part, wk.cap[4], (size_t)pmc_chunks(n_old) * n_new);
+    grow(&wk.part, wk.cap[4], (size_t)pmc_chunks(n_new, n_old) * n_new);
     if (r == PCS_OK && !wk.stream) {
         const hipError_t e = hipStreamCreateWithFlags(&wk.stream, hipStreamNonBlocking);
         if (e != hipSuccess) r = hip_error(e, "pcs_pmc_weights stream");

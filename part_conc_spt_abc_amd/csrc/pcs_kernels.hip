@@ -3094,14 +3094,16 @@ __global__ void selftest_copy_kernel(const uint4* __restrict__ src, uint4* __res
 
 // pmc-standard importance kernel sums (src/gpu/detail/simulation_impl.inl:832-871):
 // wsum[j] = sum_i w_old[i] exp(-1/2 sum_p ((x_new[p][j] - x_old[p][i]) / tau_p)^2),
-// inputs pre-divided by tau. The old members are split into chunks of
-// kPmcChunk (a 2D grid: new members x chunks, so that a large population fills
-// the GPU); a block stages 256 old members of its chunk at a time in LDS and
-// each thread sums them for its new member; pmc_reduce_kernel adds a new
-// member's chunk sums in chunk order. The order of every sum depends only on
-// the sizes, so results are reproducible.
+// inputs pre-divided by tau. A 2D grid: blocks of new members x chunks of old
+// ones; pmc_reduce_kernel adds a new member's chunk sums in a fixed order. The
+// order of every sum depends only on the sizes, so results are reproducible.
+// Bound by FP64 instructions. The old members are the same for every lane, so
+// their rows come through scalar loads straight into the multiply-adds'
+// scalar operands (staged in LDS and read back lane by lane, 7 broadcasts a
+// pair at 6 parameters, the LDS was the bound), and a lane takes kPmcJ new
+// members, each loaded row serving both.
 constexpr int kPmcMaxP = 3 * PCS_MAX_SPECIES;
-constexpr uint32_t kPmcChunk = 4096;
+constexpr uint32_t kPmcBlock = 128, kPmcJ = 2;
 
 // 2^(j/64), j = 0..63, rounded to nearest FP64 (fit_math_coeffs.py), and ln2/64
 // split into a head of 35 significant bits (k * head is exact for |k| < 2^18)
@@ -3127,68 +3129,83 @@ __constant__ double kExp2Tab64[64] = {
 constexpr double kLn2d64Hi = 0x1.62e42fefc0000p-7, kLn2d64Lo = -0x1.c610ca86c3899p-43;
 constexpr double k64dLn2 = 0x1.71547652b82fep+6;
 
-// e^y for y <= 0, tab = kExp2Tab64 in LDS: y = (64 e + j) ln2 / 64 + r with
-// k = 64 e + j = rint(64 y / ln2) (Cody-Waite), |r| <= ln2 / 128, e^r by its
-// Taylor series to degree 5 (remainder below 4e-17 relative), then
-// 2^(j/64) e^r scaled by 2^e; within 3 ulp. y is clamped at -800, where the
-// result has long underflowed to 0.
-__device__ __forceinline__ double exp_nonpos(double y, const double* tab)
+// e^y for y = -s/2, s >= 0, tab = kExp2Tab64 in LDS: y = (64 e + j) ln2 / 64 + r
+// with k = 64 e + j = rint(64 y / ln2) (the addition of 1.5 2^52 rounds, and
+// leaves k in the low bits), Cody-Waite, |r| <= ln2 / 128 (1 + 2^-40), e^r by
+// its Taylor series to degree 5 (remainder below 4e-17 relative) in q = -2 r,
+// whose powers of two are in the coefficients, then 2^(j/64) e^r scaled by 2^e;
+// within 3 ulp. s is clamped at 1600 (and a NaN to it), where the result has
+// long underflowed to 0.
+__device__ __forceinline__ double exp_neg_half(double s, const double* tab)
 {
-    y = __builtin_fmax(y, -800.0);
-    const double k = __builtin_rint(y * k64dLn2);
-    double r = __builtin_fma(-k, kLn2d64Hi, y);
-    r = __builtin_fma(-k, kLn2d64Lo, r);
-    double p = __builtin_fma(r, 0x1.1111111111111p-7, 0x1.5555555555555p-5);
-    p = __builtin_fma(p, r, 0x1.5555555555555p-3);
-    p = __builtin_fma(p, r, 0.5);
-    p = __builtin_fma(p, r, 1.0);
-    p = __builtin_fma(p, r, 1.0);
-    const int ki = (int)k;
+    s = __builtin_fmin(s, 1600.0);
+    const double kk = __builtin_fma(s, -0.5 * k64dLn2, 0x1.8p52);
+    const int ki = (int)(uint32_t)__builtin_bit_cast(uint64_t, kk);
+    const double k = kk - 0x1.8p52;
+    double q = __builtin_fma(k, 2.0 * kLn2d64Hi, s);
+    q = __builtin_fma(k, 2.0 * kLn2d64Lo, q);
+    double p = __builtin_fma(q, -0x1.1111111111111p-12, 0x1.5555555555555p-9);
+    p = __builtin_fma(p, q, -0x1.5555555555555p-6);
+    p = __builtin_fma(p, q, 0.125);
+    p = __builtin_fma(p, q, -0.5);
+    p = __builtin_fma(p, q, 1.0);
     return __builtin_ldexp(tab[ki & 63] * p, ki >> 6);
 }
 
 // P = the number of parameter rows when it is known at compile time (1..8);
-// P = 0 reads it from p_rt (up to kPmcMaxP). Dynamic LDS: the exponential's
-// table (64 doubles), then the rows of 256 staged old members, then their
-// weights.
+// P = 0 reads it from p_rt (up to kPmcMaxP).
 template <int P>
-__global__ __launch_bounds__(256) void pmc_sums_kernel(const double* xn, uint32_t n_new, const double* xo,
-                                                       const double* w_old, uint32_t n_old, uint32_t p_rt, double* part)
+__global__ __launch_bounds__(kPmcBlock) void pmc_sums_kernel(const double* __restrict__ xn, uint32_t n_new,
+                                                             const double* __restrict__ xo,
+                                                             const double* __restrict__ w_old, uint32_t n_old,
+                                                             uint32_t p_rt, uint32_t chunk, double* __restrict__ part)
 {
     constexpr int PM = P > 0 ? P : kPmcMaxP;
-    extern __shared__ double pmc_lds[];
+    constexpr int U = P > 0 ? 4 : 1;  // old members in flight
+    __shared__ double tab[64];
     const uint32_t np = P > 0 ? (uint32_t)P : p_rt;
     const uint32_t tid = threadIdx.x;
-    const uint32_t j = blockIdx.x * 256u + tid;
-    const uint32_t i_lo = blockIdx.y * kPmcChunk, i_hi = min(n_old, i_lo + kPmcChunk);
-    double* tab = pmc_lds;
-    double* sx = pmc_lds + 64;
-    double* shw = sx + (size_t)np * 256u;
-    if (tid < 64u) tab[tid] = kExp2Tab64[tid];  // first read after the loop's barrier
-    double x[PM];
+    const uint32_t j0 = blockIdx.x * (kPmcBlock * kPmcJ) + tid;
+    const uint32_t i_lo = blockIdx.y * chunk, i_hi = min(n_old, i_lo + chunk);
+    if (tid < 64u) tab[tid] = kExp2Tab64[tid];
+    __syncthreads();
+    double x[kPmcJ][PM], acc[kPmcJ];
 #pragma unroll
-    for (int p = 0; p < PM; ++p) x[p] = ((uint32_t)p < np && j < n_new) ? xn[(uint64_t)p * n_new + j] : 0.0;
-    double acc = 0.0;
-    for (uint32_t t0 = i_lo; t0 < i_hi; t0 += 256u) {
-        const uint32_t i = t0 + tid;
-        for (uint32_t p = 0; p < np; ++p) sx[p * 256u + tid] = i < i_hi ? xo[(uint64_t)p * n_old + i] : 0.0;
-        shw[tid] = i < i_hi ? w_old[i] : 0.0;
-        __syncthreads();
-        const uint32_t m = min(256u, i_hi - t0);
-        for (uint32_t ii = 0; ii < m; ++ii) {
-            double s2 = 0.0;
+    for (uint32_t c = 0; c < kPmcJ; ++c) {
+        const uint32_t j = j0 + c * kPmcBlock;
+        acc[c] = 0.0;
+#pragma unroll
+        for (int p = 0; p < PM; ++p) x[c][p] = ((uint32_t)p < np && j < n_new) ? xn[(uint64_t)p * n_new + j] : 0.0;
+    }
+    auto add = [&](uint32_t i, uint32_t n) {
+#pragma unroll
+        for (uint32_t u = 0; u < (uint32_t)U; ++u) {
+            if (u >= n) break;
+            const double w = w_old[i + u];
+            double s2[kPmcJ] = {};
 #pragma unroll
             for (int p = 0; p < PM; ++p) {
                 if (P > 0 || (uint32_t)p < np) {
-                    const double d = x[p] - sx[p * 256u + ii];
-                    s2 = __builtin_fma(d, d, s2);
+                    const double o = xo[(uint64_t)p * n_old + i + u];
+#pragma unroll
+                    for (uint32_t c = 0; c < kPmcJ; ++c) {
+                        const double d = x[c][p] - o;
+                        s2[c] = __builtin_fma(d, d, s2[c]);
+                    }
                 }
             }
-            acc = __builtin_fma(shw[ii], exp_nonpos(-0.5 * s2, tab), acc);
+#pragma unroll
+            for (uint32_t c = 0; c < kPmcJ; ++c) acc[c] = __builtin_fma(w, exp_neg_half(s2[c], tab), acc[c]);
         }
-        __syncthreads();
+    };
+    uint32_t i = i_lo;
+    for (; i + (uint32_t)U <= i_hi; i += (uint32_t)U) add(i, U);
+    for (; i < i_hi; ++i) add(i, 1u);
+#pragma unroll
+    for (uint32_t c = 0; c < kPmcJ; ++c) {
+        const uint32_t j = j0 + c * kPmcBlock;
+        if (j < n_new) part[(uint64_t)blockIdx.y * n_new + j] = acc[c];
     }
-    if (j < n_new) part[(uint64_t)blockIdx.y * n_new + j] = acc;
 }
 
 // Cumulative weights in member order: the same FP64 sums as a sequential
@@ -3266,13 +3283,47 @@ __global__ void pmc_reduce_kernel(const double* part, uint32_t n_new, uint32_t c
     const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= n_new) return;
     double s = 0.0;
-    for (uint32_t c = 0; c < chunks; ++c) s += part[(uint64_t)c * n_new + j];
+    uint32_t c = 0;
+    for (; c + 16u <= chunks; c += 16u) {  // loads of 16 chunks in flight, added in pairs
+        double v[16];
+#pragma unroll
+        for (uint32_t u = 0; u < 16u; ++u) v[u] = part[(uint64_t)(c + u) * n_new + j];
+#pragma unroll
+        for (uint32_t h = 8u; h > 0u; h /= 2u) {
+#pragma unroll
+            for (uint32_t u = 0; u < h; ++u) v[u] += v[u + h];
+        }
+        s += v[0];
+    }
+    for (; c < chunks; ++c) s += part[(uint64_t)c * n_new + j];
     wsum[j] = s;
 }
 
 // ---------------------------------------------------------------- launchers
 
-uint32_t pmc_chunks(uint32_t n_old) { return n_old ? (n_old + kPmcChunk - 1u) / kPmcChunk : 1u; }
+// Old members a chunk: 4,096, halved while there are fewer than 16 waves a
+// SIMD and fewer than 256 chunks (pmc_reduce_kernel goes through a member's
+// chunk sums one after another: 300 new against 50,000 old members in chunks
+// of 128, 47 us and 15 to add; of 32, 35 and 49), down to 32 (2,000 members:
+// chunks of 128 34 us, of 64 19, of 32 12). Kernel sums at 6 parameters,
+// chunks of 4,096 staged in LDS before: 2,000 members 203 -> 12 us, 20,000
+// 665 -> 369 us, 100,000 9.86 -> 8.71 ms; 9,000 at 9 parameters 2.18 -> 0.27 ms.
+static uint32_t pmc_chunk(uint32_t n_new, uint32_t n_old)
+{
+    const uint64_t waves = (kPmcBlock / kWave) * (uint64_t)((n_new + kPmcBlock * kPmcJ - 1u) / (kPmcBlock * kPmcJ));
+    uint32_t chunk = 4096u;
+    for (; chunk > 32u; chunk /= 2u) {
+        const uint32_t chunks = (n_old + chunk - 1u) / chunk;
+        if (chunks >= 256u || waves * chunks >= 16384u) break;
+    }
+    return chunk;
+}
+
+uint32_t pmc_chunks(uint32_t n_new, uint32_t n_old)
+{
+    const uint32_t chunk = pmc_chunk(n_new, n_old);
+    return n_old ? (n_old + chunk - 1u) / chunk : 1u;
+}
 
 hipError_t launch_pmc_sums(const double* xn, uint32_t n_new, const double* xo, const double* w_old, uint32_t n_old,
                            uint32_t P, double* part, double* wsum, hipStream_t s)
@@ -3280,24 +3331,25 @@ hipError_t launch_pmc_sums(const double* xn, uint32_t n_new, const double* xo, c
     (void)hipGetLastError();  // report only this launch's error
     if (n_new == 0) return hipSuccess;
     if (P == 0 || P > (uint32_t)kPmcMaxP) return hipErrorInvalidValue;
-    const uint32_t chunks = pmc_chunks(n_old);
-    const dim3 g((n_new + 255u) / 256u, chunks);
-    const size_t lds = (64u + ((size_t)P + 1u) * 256u) * sizeof(double);
-    const dim3 b(256);
+    const uint32_t chunk = pmc_chunk(n_new, n_old), chunks = pmc_chunks(n_new, n_old);
+    const dim3 g((n_new + kPmcBlock * kPmcJ - 1u) / (kPmcBlock * kPmcJ), chunks), b(kPmcBlock);
+    auto run = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, g, b, 0, s, xn, n_new, xo, w_old, n_old, P, chunk, part);
+    };
     switch (P) {
-    case 1: hipLaunchKernelGGL(pmc_sums_kernel<1>, g, b, lds, s, xn, n_new, xo, w_old, n_old, P, part); break;
-    case 2: hipLaunchKernelGGL(pmc_sums_kernel<2>, g, b, lds, s, xn, n_new, xo, w_old, n_old, P, part); break;
-    case 3: hipLaunchKernelGGL(pmc_sums_kernel<3>, g, b, lds, s, xn, n_new, xo, w_old, n_old, P, part); break;
-    case 4: hipLaunchKernelGGL(pmc_sums_kernel<4>, g, b, lds, s, xn, n_new, xo, w_old, n_old, P, part); break;
-    case 5: hipLaunchKernelGGL(pmc_sums_kernel<5>, g, b, lds, s, xn, n_new, xo, w_old, n_old, P, part); break;
-    case 6: hipLaunchKernelGGL(pmc_sums_kernel<6>, g, b, lds, s, xn, n_new, xo, w_old, n_old, P, part); break;
-    case 7: hipLaunchKernelGGL(pmc_sums_kernel<7>, g, b, lds, s, xn, n_new, xo, w_old, n_old, P, part); break;
-    case 8: hipLaunchKernelGGL(pmc_sums_kernel<8>, g, b, lds, s, xn, n_new, xo, w_old, n_old, P, part); break;
-    default: hipLaunchKernelGGL(pmc_sums_kernel<0>, g, b, lds, s, xn, n_new, xo, w_old, n_old, P, part); break;
+    case 1: run(pmc_sums_kernel<1>); break;
+    case 2: run(pmc_sums_kernel<2>); break;
+    case 3: run(pmc_sums_kernel<3>); break;
+    case 4: run(pmc_sums_kernel<4>); break;
+    case 5: run(pmc_sums_kernel<5>); break;
+    case 6: run(pmc_sums_kernel<6>); break;
+    case 7: run(pmc_sums_kernel<7>); break;
+    case 8: run(pmc_sums_kernel<8>); break;
+    default: run(pmc_sums_kernel<0>); break;
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(pmc_reduce_kernel, dim3((n_new + 255u) / 256u), dim3(256), 0, s, part, n_new, chunks, wsum);
+    hipLaunchKernelGGL(pmc_reduce_kernel, dim3((n_new + 63u) / 64u), dim3(64), 0, s, part, n_new, chunks, wsum);
     return hipGetLastError();
 }
 
