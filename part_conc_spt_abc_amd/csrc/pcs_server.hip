@@ -109,17 +109,12 @@ struct Group {
     bool busy = false;
     hipStream_t stream = nullptr;
     hipEvent_t done = nullptr;
-    // device tables of this group; one tile table per model class, so the
-    // walks of every class present are issued back to back
-    DevProp* d_props = nullptr;
-    uint32_t *d_vframes = nullptr, *d_vparticles = nullptr, *d_vprop = nullptr;
-    uint32_t* d_vtile[kClasses] = {};
-    uint32_t* d_count = nullptr;
+    // tables of this group, one behind the other in device memory and in
+    // pinned staging, packed to the group's sizes so that one copy uploads them
+    // (launch_group)
+    unsigned char *d_tab = nullptr, *h_tab = nullptr;
     DistScratch* d_dscratch = nullptr;
-    // pinned host staging (uploads) and results (written by the distance kernel)
-    DevProp* h_props = nullptr;
-    uint32_t *h_vframes = nullptr, *h_vparticles = nullptr, *h_vprop = nullptr;
-    uint32_t* h_vtile[kClasses] = {};
+    // pinned host results (written by the distance kernel)
     double* h_dist = nullptr;
     uint64_t* h_exact = nullptr;
     uint32_t* h_tracks = nullptr;
@@ -206,23 +201,23 @@ hipError_t dmalloc(T** p, size_t n) { return hipMalloc((void**)p, std::max<size_
 template <typename T>
 hipError_t hmalloc(T** p, size_t n) { return hipHostMalloc((void**)p, std::max<size_t>(n, 1) * sizeof(T), hipHostMallocDefault); }
 
+// A launch group's tables: simulations, their record counters (uploaded as
+// zeros), video lengths, particle counts and owners, and a tile table for each
+// model class present, so that the walks of every class are issued back to back.
+size_t table_bytes(size_t n, size_t nv, size_t classes)
+{
+    return n * (sizeof(DevProp) + 4u) + (3u * nv + classes * (nv + 1u)) * 4u;
+}
+
 hipError_t group_alloc(Group& g, uint32_t max_props, uint32_t max_videos)
 {
     hipError_t e = hipStreamCreateWithFlags(&g.stream, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipEventCreateWithFlags(&g.done, hipEventDisableTiming);
-    if (e == hipSuccess) e = dmalloc(&g.d_props, max_props);
-    if (e == hipSuccess) e = dmalloc(&g.d_vframes, max_videos);
-    if (e == hipSuccess) e = dmalloc(&g.d_vparticles, max_videos);
-    if (e == hipSuccess) e = dmalloc(&g.d_vprop, max_videos);
-    for (int k = 0; k < kClasses && e == hipSuccess; ++k) e = dmalloc(&g.d_vtile[k], max_videos + 1);
-    if (e == hipSuccess) e = dmalloc(&g.d_count, max_props);
+    const size_t tab = table_bytes(max_props, max_videos, kClasses);
+    if (e == hipSuccess) e = dmalloc(&g.d_tab, tab);
+    if (e == hipSuccess) e = hmalloc(&g.h_tab, tab);
     if (e == hipSuccess) e = dmalloc(&g.d_dscratch, 1);
     if (e == hipSuccess) e = hipMemset(g.d_dscratch, 0, sizeof(DistScratch));
-    if (e == hipSuccess) e = hmalloc(&g.h_props, max_props);
-    if (e == hipSuccess) e = hmalloc(&g.h_vframes, max_videos);
-    if (e == hipSuccess) e = hmalloc(&g.h_vparticles, max_videos);
-    if (e == hipSuccess) e = hmalloc(&g.h_vprop, max_videos);
-    for (int k = 0; k < kClasses && e == hipSuccess; ++k) e = hmalloc(&g.h_vtile[k], max_videos + 1);
     if (e == hipSuccess) e = hmalloc(&g.h_dist, max_props);
     if (e == hipSuccess) e = hmalloc(&g.h_exact, max_props);
     if (e == hipSuccess) e = hmalloc(&g.h_tracks, max_props);
@@ -233,16 +228,12 @@ hipError_t group_alloc(Group& g, uint32_t max_props, uint32_t max_videos)
 void group_free(Group& g)
 {
     if (g.stream) hipStreamSynchronize(g.stream);
-    void* dev[] = {g.d_props, g.d_vframes, g.d_vparticles, g.d_vprop, g.d_count, g.d_dscratch};
+    void* dev[] = {g.d_tab, g.d_dscratch};
     for (void* p : dev)
         if (p) hipFree(p);
-    void* host[] = {g.h_props, g.h_vframes, g.h_vparticles, g.h_vprop, g.h_dist, g.h_exact, g.h_tracks, g.h_status};
+    void* host[] = {g.h_tab, g.h_dist, g.h_exact, g.h_tracks, g.h_status};
     for (void* p : host)
         if (p) hipHostFree(p);
-    for (int k = 0; k < kClasses; ++k) {
-        if (g.d_vtile[k]) hipFree(g.d_vtile[k]);
-        if (g.h_vtile[k]) hipHostFree(g.h_vtile[k]);
-    }
     if (g.done) hipEventDestroy(g.done);
     if (g.stream) hipStreamDestroy(g.stream);
     g = Group{};
@@ -275,58 +266,73 @@ DevProp make_prop(const pcs_server* s, const Pending& p, uint32_t first_video, u
 int launch_group(pcs_server* s, Group& g, std::vector<Pending>& batch, std::vector<uint64_t>& offs)
 {
     const uint32_t n = (uint32_t)batch.size();
-    uint32_t nv = 0;
     g.arena_off.assign(offs.begin(), offs.end());
-    uint32_t n_de_max = 1, n_k_max = 1;
+    uint32_t n_videos = 0, n_de_max = 1, n_k_max = 1;
     uint32_t classes = 0;  // bit model_class() present
+    for (const Pending& p : batch) {
+        const pcs_system& sy = s->systems[p.req.sys_id].sys;
+        n_videos += p.req.n_videos;
+        n_de_max = std::max(n_de_max, sy.n_de);
+        n_k_max = std::max(n_k_max, sy.n_k);
+        classes |= 1u << model_class(sy);
+    }
+    // the tables' places in h_tab and, the same, in d_tab
+    DevProp* props = reinterpret_cast<DevProp*>(g.h_tab);
+    uint32_t* count = reinterpret_cast<uint32_t*>(props + n);
+    uint32_t *vframes = count + n, *vparticles = vframes + n_videos, *vprop = vparticles + n_videos;
+    uint32_t* vtile[kClasses] = {};
+    uint32_t* end = vprop + n_videos;
+    for (uint32_t k = 0; k < (uint32_t)kClasses; ++k) {
+        if (!(classes & (1u << k))) continue;
+        vtile[k] = end;
+        end += n_videos + 1u;
+    }
+    const size_t bytes = table_bytes(n, n_videos, (size_t)__builtin_popcount(classes));
+    auto dev = [&g](auto* h) {
+        return reinterpret_cast<decltype(h)>(g.d_tab + (reinterpret_cast<unsigned char*>(h) - g.h_tab));
+    };
+    uint32_t nv = 0;
     uint32_t tiles[kClasses] = {0, 0, 0, 0};
     for (uint32_t i = 0; i < n; ++i) {
         const Pending& p = batch[i];
-        const pcs_system& sy = s->systems[p.req.sys_id].sys;
-        const uint32_t cls = model_class(sy);
-        g.h_props[i] = make_prop(s, p, nv, offs[i]);
+        const uint32_t cls = model_class(s->systems[p.req.sys_id].sys);
+        props[i] = make_prop(s, p, nv, offs[i]);
+        count[i] = 0u;
         for (uint32_t v = 0; v < p.req.n_videos; ++v, ++nv) {
-            g.h_vframes[nv] = p.frames[v];
-            g.h_vparticles[nv] = p.particles[v];
-            g.h_vprop[nv] = i;
+            vframes[nv] = p.frames[v];
+            vparticles[nv] = p.particles[v];
+            vprop[nv] = i;
             // tile tables: the videos of other classes have no tiles in this one
             for (uint32_t k = 0; k < (uint32_t)kClasses; ++k) {
-                g.h_vtile[k][nv] = tiles[k];
+                if (vtile[k]) vtile[k][nv] = tiles[k];
                 if (k == cls) tiles[k] += (p.particles[v] + 63u) / 64u;
             }
         }
-        n_de_max = std::max(n_de_max, sy.n_de);
-        n_k_max = std::max(n_k_max, sy.n_k);
-        classes |= 1u << cls;
     }
+    for (uint32_t k = 0; k < (uint32_t)kClasses; ++k)
+        if (vtile[k]) vtile[k][nv] = tiles[k];
     g.reqs.clear();
     for (Pending& p : batch) g.reqs.push_back(std::move(p));
     g.n = n;
     hipStream_t st = g.stream;
-    hipError_t e = hipMemcpyAsync(g.d_props, g.h_props, n * sizeof(DevProp), hipMemcpyHostToDevice, st);
-    if (e == hipSuccess) e = hipMemcpyAsync(g.d_vframes, g.h_vframes, nv * 4, hipMemcpyHostToDevice, st);
-    if (e == hipSuccess) e = hipMemcpyAsync(g.d_vparticles, g.h_vparticles, nv * 4, hipMemcpyHostToDevice, st);
-    if (e == hipSuccess) e = hipMemcpyAsync(g.d_vprop, g.h_vprop, nv * 4, hipMemcpyHostToDevice, st);
-    if (e == hipSuccess) e = launch_reset(g.d_count, n, nullptr, st);
+    // One copy brings all tables and the zeroed counters.
+    hipError_t e = hipMemcpyAsync(g.d_tab, g.h_tab, bytes, hipMemcpyHostToDevice, st);
     // One walk launch per (detection, boundary) class present, each over its
     // own tile table.
     for (uint32_t cls = 0; cls < (uint32_t)kClasses && e == hipSuccess; ++cls) {
         if (!(classes & (1u << cls))) continue;
-        g.h_vtile[cls][nv] = tiles[cls];
-        e = hipMemcpyAsync(g.d_vtile[cls], g.h_vtile[cls], (nv + 1) * 4, hipMemcpyHostToDevice, st);
-        if (e != hipSuccess) break;
         WalkArgs a{};
         a.sys = s->d_sys;
-        a.props = g.d_props;
-        a.vframes = g.d_vframes;
-        a.vparticles = g.d_vparticles;
-        a.vprop = g.d_vprop;
-        a.vtile = g.d_vtile[cls];
+        a.props = dev(props);
+        a.vframes = dev(vframes);
+        a.vparticles = dev(vparticles);
+        a.vprop = dev(vprop);
+        a.vtile = dev(vtile[cls]);
         a.n_videos = nv;
         a.tile_lo = 0;
         a.tile_hi = tiles[cls];
         a.stage_cap = 256;
-        a.rec_count = g.d_count;
+        a.rec_count = dev(count);
         a.seed = s->d_zero_seed;
         a.tile_counter = nullptr;
         e = launch_walk(a, 1, 4, false, 0, (cls & 2u) != 0, (cls & 1u) != 0, st);
@@ -334,10 +340,10 @@ int launch_group(pcs_server* s, Group& g, std::vector<Pending>& batch, std::vect
     if (e == hipSuccess) {
         DistArgs d{};
         d.sys = s->d_sys;
-        d.props = g.d_props;
+        d.props = dev(props);
         d.prop_lo = 0;
         d.n_props = n;
-        d.rec_count = g.d_count;
+        d.rec_count = dev(count);
         d.dist = g.h_dist;
         d.exact = g.h_exact;
         d.tracks = g.h_tracks;
