@@ -151,6 +151,13 @@ struct pcs_ctx {
     pcs_batch* oneshot = nullptr;
 };
 
+// What every batch has on the device, in one allocation.
+struct FixedState {
+    DistScratch dist[1 + PCS_PLAIN_STREAMS];  // of the batch stream, then of each plain stream
+    uint64_t seed;
+    uint32_t tile_counter;
+};
+
 struct pcs_batch {
     pcs_ctx* ctx = nullptr;
     hipStream_t stream = nullptr;
@@ -171,11 +178,12 @@ struct pcs_batch {
     // device
     DevProp* d_props = nullptr;
     uint32_t *d_vframes = nullptr, *d_vparticles = nullptr, *d_vprop = nullptr, *d_vtile = nullptr;
-    uint32_t *d_rec = nullptr, *d_srt = nullptr, *d_count = nullptr, *d_tile_counter = nullptr;
+    uint32_t *d_rec = nullptr, *d_srt = nullptr, *d_count = nullptr;
     // Results: written by the distance kernel straight into pinned host memory
     // for up to kHostResults simulations (a read is then one wait; copying
     // the arrays back cost 60 us), into device memory above.
     bool host_res = false;
+    unsigned char* results = nullptr;  // the allocation of the arrays below
     uint32_t* d_tracks = nullptr;
     double* d_dist = nullptr;
     uint64_t* d_exact = nullptr;
@@ -185,7 +193,10 @@ struct pcs_batch {
     uint32_t *d_hist = nullptr, *h_hist = nullptr;
     size_t cap_hist = 0;
     bool plan_ran = false;  // the present plan has run once (the graph pays from the second run on)
-    uint64_t* d_seed = nullptr;
+    FixedState* d_fixed = nullptr;
+    uint64_t* d_seed = nullptr;          // in d_fixed, like the next two
+    uint32_t* d_tile_counter = nullptr;
+    DistScratch* d_dscratch = nullptr;
     uint64_t* h_seed = nullptr;  // pinned
     size_t cap_props = 0, cap_videos = 0, cap_arena = 0;
     // device-planned batch (pcs_batch_propose): the proposal records, the
@@ -235,8 +246,6 @@ struct pcs_batch {
     int last_mode = -1;
     bool ran = false;
     uint32_t reruns = 0;
-    // distance scratch: of the batch stream, then of each plain stream
-    DistScratch* d_dscratch = nullptr;
 };
 
 namespace {
@@ -275,32 +284,30 @@ constexpr uint64_t kOneshotKeep = 4u << 20;  // records of a kept pcs_simulate b
 
 void free_results(pcs_batch* b)
 {
-    void* ptrs[] = {b->d_tracks, b->d_dist, b->d_exact, b->d_status};
-    for (void* q : ptrs)
-        if (q) b->host_res ? hipHostFree(q) : hipFree(q);
-    b->d_tracks = nullptr;
+    if (b->results) b->host_res ? hipHostFree(b->results) : hipFree(b->results);
+    b->results = nullptr;
     b->d_dist = nullptr;
     b->d_exact = nullptr;
+    b->d_tracks = nullptr;
     b->d_status = nullptr;
 }
 
-// Result arrays of n simulations (the stream is idle).
+// Result arrays of n simulations, in one allocation (the stream is idle).
 int alloc_results(pcs_batch* b, uint32_t n)
 {
     free_results(b);
     b->host_res = n <= kHostResults;
-    if (!b->host_res) {
-        PCS_TRY(dev_alloc(&b->d_tracks, n));
-        PCS_TRY(dev_alloc(&b->d_dist, n));
-        PCS_TRY(dev_alloc(&b->d_exact, n));
-        return dev_alloc(&b->d_status, n);
+    const size_t m = n ? n : 1, bytes = m * (8u + 8u + 4u + 4u);
+    const hipError_t e = b->host_res ? hipHostMalloc((void**)&b->results, bytes, hipHostMallocDefault)
+                                     : hipMalloc((void**)&b->results, bytes);
+    if (e != hipSuccess) {
+        b->results = nullptr;
+        return set_error(PCS_ENOMEM, "results of %u simulations: %s", n, hipGetErrorString(e));
     }
-    const size_t m = n ? n : 1;
-    hipError_t e = hipHostMalloc((void**)&b->d_tracks, m * 4u, hipHostMallocDefault);
-    if (e == hipSuccess) e = hipHostMalloc((void**)&b->d_dist, m * 8u, hipHostMallocDefault);
-    if (e == hipSuccess) e = hipHostMalloc((void**)&b->d_exact, m * 8u, hipHostMallocDefault);
-    if (e == hipSuccess) e = hipHostMalloc((void**)&b->d_status, m * 4u, hipHostMallocDefault);
-    if (e != hipSuccess) return set_error(PCS_ENOMEM, "hipHostMalloc (results of %u simulations): %s", n, hipGetErrorString(e));
+    b->d_dist = reinterpret_cast<double*>(b->results);
+    b->d_exact = reinterpret_cast<uint64_t*>(b->d_dist + m);
+    b->d_tracks = reinterpret_cast<uint32_t*>(b->d_exact + m);
+    b->d_status = reinterpret_cast<int32_t*>(b->d_tracks + m);
     return PCS_OK;
 }
 
@@ -887,11 +894,13 @@ int pcs_batch_create(pcs_ctx* c, pcs_batch** out)
     for (int i = 0; i < 4 && e == hipSuccess; ++i) e = hipEventCreate(&b->ev[i]);
     if (e == hipSuccess) e = hipHostMalloc((void**)&b->h_seed, sizeof(uint64_t), hipHostMallocDefault);
     int r = e == hipSuccess ? PCS_OK : hip_error(e, "pcs_batch_create");
-    if (r == PCS_OK) r = dev_alloc(&b->d_seed, 1);
-    if (r == PCS_OK) r = dev_alloc(&b->d_tile_counter, 1);
-    if (r == PCS_OK) r = dev_alloc(&b->d_dscratch, 1 + PCS_PLAIN_STREAMS);
+    if (r == PCS_OK) r = dev_alloc(&b->d_fixed, 1);
     if (r == PCS_OK) {
-        e = hipMemset(b->d_dscratch, 0, (1 + PCS_PLAIN_STREAMS) * sizeof(DistScratch));
+        b->d_seed = &b->d_fixed->seed;
+        b->d_tile_counter = &b->d_fixed->tile_counter;
+        b->d_dscratch = b->d_fixed->dist;
+        // the plain streams fork from the batch stream
+        e = hipMemsetAsync(b->d_fixed, 0, sizeof(FixedState), b->stream);
         if (e != hipSuccess) r = hip_error(e, "pcs_batch_create");
     }
     if (r != PCS_OK) {
@@ -912,9 +921,9 @@ int pcs_batch_destroy(pcs_batch* b)
     if (b->wstream) hipStreamSynchronize(b->wstream);
     destroy_graph(b);
     void* ptrs[] = {b->d_props, b->d_vframes, b->d_vparticles, b->d_vprop, b->d_vtile, b->d_rec, b->d_srt,
-                    b->d_rec2, b->d_srt2, b->d_count, b->d_tile_counter, b->d_hist, b->d_vorder, b->d_otile,
-                    b->d_seed, b->d_in, b->d_theta_pop, b->d_cumw, b->d_theta_new, b->d_totals, b->d_bsums, b->d_wpop,
-                    b->d_xn, b->d_xo, b->d_wsum, b->d_part, b->d_dscratch};
+                    b->d_rec2, b->d_srt2, b->d_count, b->d_fixed, b->d_hist, b->d_vorder, b->d_otile,
+                    b->d_in, b->d_theta_pop, b->d_cumw, b->d_theta_new, b->d_totals, b->d_bsums, b->d_wpop,
+                    b->d_xn, b->d_xo, b->d_wsum, b->d_part};
     for (void* p : ptrs)
         if (p) hipFree(p);
     free_results(b);

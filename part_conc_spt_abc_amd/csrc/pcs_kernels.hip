@@ -9,6 +9,9 @@
 //                    and appended to the proposal's HBM record slice with one
 //                    atomic per flush (replaces the per-track global atomicInc
 //                    of src/gpu/cusim/histogram2d.inl:98-106).
+//   walk_group_kernel  few tiles: one tile by a workgroup of 11 waves, eight
+//                    making the random numbers, two moving the particles, one
+//                    keeping their tracks.
 //   distance_kernel  one workgroup per proposal: counting sort of the records
 //                    by row (LDS row counters; the records are read once and
 //                    held in registers, the sorted 16-bit bins kept in LDS
@@ -21,6 +24,8 @@
 //                    table, whose rows are loaded ahead. Replaces K_distance
 //                    (src/gpu/cusim/kernel-distance.inl:81-241), a single 32x32
 //                    block that scanned the whole dense histogram in FP32.
+//   distance_split_kernel  the same distance of few simulations, the rows split
+//                    over several workgroups and their waves.
 //   serve_loop_kernel  device-resident request loop: one admitter wave copies
 //                    requests from a ring in pinned host memory into HBM slots,
 //                    the other groups take their tiles, walk them and run the
