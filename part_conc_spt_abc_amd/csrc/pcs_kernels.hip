@@ -857,7 +857,8 @@ __global__ __launch_bounds__(256) void walk_kernel(WalkArgs a)
             process_tile<PPL, GAUSS, ZREF, TRACKS>(a, t, st, tab, k0, k1);
         }
     } else {
-        const uint32_t t = a.tile_lo + blockIdx.x * wpg + wave;
+        // (taken wave-uniform: 59 VGPRs, with the tile's data a lane each 79)
+        const uint32_t t = uniform(a.tile_lo + blockIdx.x * wpg + wave);
         if (t < a.tile_hi) process_tile<PPL, GAUSS, ZREF, TRACKS>(a, t, st, tab, k0, k1);
     }
 }
