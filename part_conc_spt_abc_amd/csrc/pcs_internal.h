@@ -104,7 +104,8 @@ struct WalkArgs {
     uint32_t stage_cap;         // LDS records per wave
     uint32_t* rec_count;        // per proposal, atomically bumped
     const uint64_t* seed;       // device-resident Philox key
-    uint32_t* tile_counter;     // persistent form: next tile (relative to tile_lo)
+    uint32_t* tile_counter;     // persistent form: tiles taken past the waves' own first ones
+    uint32_t own_groups;        // persistent form: workgroups whose waves own a first tile (launch_walk)
     const uint64_t* tile_total; // persistent form, nullable: tiles planned on the device (caps tile_hi)
 };
 

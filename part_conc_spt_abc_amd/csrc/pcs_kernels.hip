@@ -849,10 +849,19 @@ __global__ __launch_bounds__(256) void walk_kernel(WalkArgs a)
     if (PERSIST) {
         // tiles planned on the device end the range where the plan says
         const uint32_t hi = a.tile_total ? (uint32_t)min((uint64_t)a.tile_hi, *a.tile_total) : a.tile_hi;
+        // The first tile of a wave of the first own_groups workgroups is its
+        // own; the counter gives the ones after.
+        const uint32_t own = a.own_groups * wpg;
+        uint32_t t = uniform(blockIdx.x * wpg + wave);
+        bool claim = t >= own;
         for (;;) {
-            uint32_t t = 0u;
-            if (lane_id() == 0u) t = atomicAdd(a.tile_counter, 1u);
-            t = uniform(t) + a.tile_lo;
+            if (claim) {
+                uint32_t c = 0u;
+                if (lane_id() == 0u) c = atomicAdd(a.tile_counter, 1u);
+                t = own + uniform(c);
+            }
+            claim = true;
+            t += a.tile_lo;
             if (t >= hi) break;
             process_tile<PPL, GAUSS, ZREF, TRACKS>(a, t, st, tab, k0, k1);
         }
@@ -3405,11 +3414,40 @@ static uint32_t device_cus()
     return (uint32_t)n;
 }
 
+// Workgroups of a walk kernel that run at once, per (device, kernel, threads,
+// LDS), found once: the occupancy query does not touch a stream.
+static uint32_t resident_groups(const void* fn, int threads, size_t shmem)
+{
+    static std::mutex mu;
+    static std::map<std::tuple<int, const void*, int, size_t>, uint32_t> memo;
+    int dev = 0, n = 0;
+    (void)hipGetDevice(&dev);
+    std::lock_guard<std::mutex> lk(mu);
+    const auto key = std::make_tuple(dev, fn, threads, shmem);
+    auto it = memo.find(key);
+    if (it != memo.end()) return it->second;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, fn, threads, shmem) != hipSuccess || n < 0) {
+        (void)hipGetLastError();
+        n = 0;
+    }
+    const uint32_t groups = (uint32_t)n * device_cus();
+    memo.emplace(key, groups);
+    return groups;
+}
+
 template <int PPL, bool PERSIST, bool GAUSS, bool ZREF>
-static hipError_t launch_walk_t(const WalkArgs& a, int wpg, uint32_t grid, hipStream_t s)
+static hipError_t launch_walk_t(WalkArgs a, int wpg, uint32_t grid, hipStream_t s)
 {
     (void)hipGetLastError();  // report only this launch's error
     const size_t shmem = ((size_t)wpg * a.stage_cap + kAngleTabFloats) * sizeof(uint32_t);
+    // First tiles without the counter, for as many workgroups as run at once
+    // (a later one's own tile would come last): thousands of waves at the
+    // counter, one behind the other, started the last of them 0.08 ms late.
+    // Walk of 7,078 tiles of 1,000 frames 0.84 -> 0.76 ms, of 50,231 4.56 ->
+    // 4.40, of 11,530 of 101 to 999 frames 0.72 -> 0.62.
+    if (PERSIST)
+        a.own_groups = std::min(grid, resident_groups(reinterpret_cast<const void*>(walk_kernel<PPL, PERSIST, GAUSS, ZREF>),
+                                                      wpg * kWave, shmem));
     hipLaunchKernelGGL((walk_kernel<PPL, PERSIST, GAUSS, ZREF>), dim3(grid), dim3(wpg * kWave), shmem, s, a);
     return hipGetLastError();
 }
