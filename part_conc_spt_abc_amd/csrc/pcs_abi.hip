@@ -85,15 +85,22 @@ void build_sat(const uint32_t* H, uint32_t n_k, uint32_t n_de, std::vector<uint3
 {
     const uint32_t pitch = sat_pitch(n_de), pad = pitch - n_de;
     S.assign((size_t)n_k * pitch, 0u);
-    maxrow = 0;
+    maxrow = most = 0;
+    if (!H) return;  // nothing observed
     uint64_t all = 0;  // observed tracks: no entry is larger, or wraps, below 2^32 of them
     for (uint32_t i = 0; i < n_k; ++i) {
-        uint64_t run = 0;
+        const uint32_t* h = H + (size_t)i * n_de;
         uint32_t* row = S.data() + (size_t)i * pitch + pad;
+        uint32_t any = 0;
+        for (uint32_t j = 0; j < n_de; ++j) any |= h[j];
+        if (any == 0) {  // most of the deep rows
+            if (i) std::copy(row - pitch, row - pitch + n_de, row);
+            continue;
+        }
+        maxrow = i;
+        uint64_t run = 0;
         for (uint32_t j = 0; j < n_de; ++j) {
-            const uint32_t h = H ? H[(size_t)i * n_de + j] : 0u;
-            if (h) maxrow = i;
-            run += h;
+            run += h[j];
             row[j] = (uint32_t)run + (i ? row[(ptrdiff_t)j - (ptrdiff_t)pitch] : 0u);
         }
         all += run;
