@@ -3475,15 +3475,16 @@ hipError_t launch_walk(const WalkArgs& a, int ppl, int wpg, bool persistent, uin
                        bool gauss, bool zref, hipStream_t s)
 {
     if (a.tile_hi <= a.tile_lo) return hipSuccess;
-    // Few tiles: a workgroup each, as long as that beats a wave each. At 1,000
-    // frames, group against wave: 4 tiles (500 frames) 41 against 205 us, 379
-    // 92 against 370, 1,510 270 against 500, 3,005 532 against 645, 4,520 770
-    // against 755; Gaussian detection at 2,000 frames 1,506 tiles 735 against
-    // 1,180, 3,005 1,420 against 1,460, 6,002 2,750 against 1,800. (A range
-    // planned on the device is not known here, and tiles of 128 particles are
-    // not the group's.)
+    // Few tiles: a workgroup each, as long as that beats a wave each: up to
+    // 6.75 tiles a CU, 3.75 with Gaussian detection. Group against wave at
+    // 1,000 frames: 4 tiles (500 frames) 41 against 205 us, 1,000 180 against
+    // 255, 1,500 260 against 298, 2,000 330 against 294, 3,500 537 against 436;
+    // Gaussian at 2,000 frames 1,000 tiles 640 against 620, 2,000 1,263 against
+    // 750; at 300 frames 1,500 tiles 88 against 100, 2,000 114 against 101. (A
+    // range planned on the device is not known here, and tiles of 128 particles
+    // are not the group's.)
     const uint32_t n_cu = device_cus();
-    if (ppl == 1 && !a.tile_total && a.tile_hi - a.tile_lo <= (gauss ? 11u : 14u) * n_cu) {
+    if (ppl == 1 && !a.tile_total && 4u * (uint64_t)(a.tile_hi - a.tile_lo) <= (gauss ? 15u : 27u) * n_cu) {
         const uint32_t grid = std::min(a.tile_hi - a.tile_lo, (gauss ? 1u : 2u) * n_cu);
         if (gauss) return zref ? launch_group_t<true, true>(a, grid, s) : launch_group_t<true, false>(a, grid, s);
         return zref ? launch_group_t<false, true>(a, grid, s) : launch_group_t<false, false>(a, grid, s);

@@ -27,7 +27,7 @@ def test_gauss_bound(gpu_lib, sigma, walls):
     f, parts = np.full(n, 40, np.uint32), np.full(n, 1000, np.uint32)
     got = []
     with Context(model) as ctx:
-        assert n * 16 > 11 * 256  # tiles, walked by groups up to 11 a CU
+        assert n * 16 > 11 * 256  # tiles: more than are walked by groups
         b = ctx.batch()
         b.load(props, f, parts)
         for mode in (_abi.PCS_MODE_BATCHED, _abi.PCS_MODE_PLAIN):
