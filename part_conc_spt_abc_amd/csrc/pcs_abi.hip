@@ -1279,14 +1279,17 @@ int pcs_batch_propose(pcs_batch* b, const pcs_prior* pr, const double* theta, co
     b->ready = false;
     b->ran = false;
     const uint32_t nv = n_trials * J;
-    bool relayout = !b->dev_planned || n_trials != b->n_props || J != b->J;
+    // The captured graph holds these buffers and sizes: it goes before any of
+    // them changes, so that a call failing further on leaves no graph that the
+    // next call of the same size would take for its own.
+    if (!b->dev_planned || n_trials != b->n_props || J != b->J) destroy_graph(b);
     if (n_trials > b->cap_props) {
+        destroy_graph(b);
         b->cap_props = 0;
         PCS_TRY(dev_alloc(&b->d_props, n_trials));
         PCS_TRY(dev_alloc(&b->d_count, n_trials));
         PCS_TRY(alloc_results(b, n_trials));
         b->cap_props = n_trials;
-        relayout = true;
     }
     if (n_trials > b->cap_in || !b->d_in) {
         b->cap_in = b->cap_new = 0;
@@ -1295,13 +1298,13 @@ int pcs_batch_propose(pcs_batch* b, const pcs_prior* pr, const double* theta, co
         b->cap_in = b->cap_new = n_trials;
     }
     if ((size_t)nv + 1u > b->cap_videos) {
+        destroy_graph(b);
         b->cap_videos = 0;
         PCS_TRY(dev_alloc(&b->d_vframes, (size_t)nv + 1u));
         PCS_TRY(dev_alloc(&b->d_vparticles, (size_t)nv + 1u));
         PCS_TRY(dev_alloc(&b->d_vprop, (size_t)nv + 1u));
         PCS_TRY(dev_alloc(&b->d_vtile, (size_t)nv + 1u));
         b->cap_videos = (size_t)nv + 1u;
-        relayout = true;
     }
     if (!resident) b->pop_resident = false;  // replaced by an uploaded population without weights
     if (!resident && (n_pop > b->cap_pop || !b->d_theta_pop)) {
@@ -1367,11 +1370,11 @@ int pcs_batch_propose(pcs_batch* b, const pcs_prior* pr, const double* theta, co
                          (unsigned long long)tot[1]);
     if (tot[0] > b->cap_arena || !b->d_rec) {
         const uint64_t cap = tot[0] + tot[0] / 8u + 1024u;
+        destroy_graph(b);
         b->cap_arena = 0;
         PCS_TRY(dev_alloc(&b->d_rec, cap));
         PCS_TRY(dev_alloc(&b->d_srt, cap));
         b->cap_arena = cap;
-        relayout = true;
         PCS_TRY(device_plan(b));
     }
     b->last_need = tot[0];
@@ -1382,7 +1385,6 @@ int pcs_batch_propose(pcs_batch* b, const pcs_prior* pr, const double* theta, co
                                    (size_t)n_trials * 8u, hipMemcpyDeviceToHost, st));
     }
     PCS_HIP(hipStreamSynchronize(st));
-    if (relayout) destroy_graph(b);
     // the point pcs_batch_pmc_weights_async starts from: the trials exist
     if (!b->wstream) {
         PCS_HIP(hipStreamCreateWithFlags(&b->wstream, hipStreamNonBlocking));

@@ -1,0 +1,54 @@
+"""A batch and a context used on after a call that failed, that was empty or
+that was unusually large: what a call leaves behind must not reach the next."""
+import numpy as np
+import pytest
+
+import cases
+from part_conc_spt_abc_amd import _abi
+from part_conc_spt_abc_amd.gpu import Context
+from part_conc_spt_abc_amd.model import prior_record
+
+pytestmark = pytest.mark.gpu
+
+
+def population(n_pop, log10c):
+    rng = np.random.default_rng(n_pop)
+    theta = np.vstack([rng.uniform(0.5, 2.5, (2, n_pop)), np.full((2, n_pop), log10c), np.full((1, n_pop), 2.0)])
+    return theta, np.cumsum(np.full(n_pop, 1.0 / n_pop)), np.array([0.1, 0.1, 0.0, 0.0, 0.1])
+
+
+def test_propose_after_a_failed_propose(gpu_lib):
+    """A batch whose graph is captured; a proposal step of more trials that is
+    refused after the buffers have grown (more than 2^32 tiles); then the same
+    number of trials, which need no larger arena. Its graph is a new one."""
+    model = cases.headline_model(n_k=60, n_de=40)
+    obs = np.zeros((60, 40), np.uint32)
+    obs[4, 7] = 3
+    few, many = 400, 20000
+    with Context(model, obs) as ctx:
+        b = ctx.batch()
+        b.propose(prior_record(model, (0.1, 5.0), (8.0, 10.0), (0.5, 4.0)), *population(50, 9.7), few,
+                  np.full((few, 1), 300, np.uint32), 3)
+        for seed in (1, 2, 3):  # direct, captured, replayed
+            b.run(seed)
+            b.read()
+        assert b.arena()[0] > 0
+        frames = np.full((many, 1), 12, np.uint32)
+        with pytest.raises(_abi.PcsError, match="more than 2\\^32 - 1") as e:
+            b.propose(prior_record(model, (0.1, 5.0), (8.0, 12.83), (0.5, 4.0)), *population(50, 12.82), many, frames, 4)
+        assert e.value.code == _abi.PCS_EINVAL
+        with pytest.raises(_abi.PcsError):
+            b.run(5)
+        pr = prior_record(model, (0.1, 5.0), (5.0, 10.0), (0.5, 4.0))
+        c = ctx.batch()
+        got = []
+        for q in (b, c):
+            q.propose(pr, *population(50, 7.0), many, frames, 6)
+            for seed in (7, 8):
+                q.run(seed)
+                _, tracks, _ = q.read()
+                got.append((tracks, q.read_exact()))
+        assert int(got[0][0].sum()) > 0
+        assert all(np.array_equal(x, y) for k in (0, 1) for x, y in zip(got[k], got[k + 2]))
+        c.close()
+        b.close()
