@@ -154,8 +154,12 @@ struct pcs_ctx {
     // caller's, and the context is freed when its last batch is destroyed.
     std::atomic<int> refs{1};
     // pcs_simulate's batch, kept from call to call while it is small (making
-    // and freeing one costs 150 us of allocations); pcs_close gives it back.
-    pcs_batch* oneshot = nullptr;
+    // and freeing one costs 150 us of allocations); pcs_close gives it back. A
+    // call takes it out for itself and puts it back if the place is still
+    // empty, so calls that overlap on a context each have a batch of their own;
+    // after pcs_close it is taken (by kClosed), and a call still running frees
+    // its batch.
+    std::atomic<pcs_batch*> oneshot{nullptr};
 };
 
 // What every batch has on the device, in one allocation.
@@ -276,6 +280,7 @@ int dev_alloc(T** p, size_t n)
 constexpr uint32_t kHostResults = 4096;
 constexpr size_t kHistKeep = 16u << 20;     // bytes
 constexpr uint64_t kOneshotKeep = 4u << 20;  // records of a kept pcs_simulate batch
+pcs_batch* const kClosed = reinterpret_cast<pcs_batch*>(alignof(pcs_batch));  // no batch
 
 #define PCS_HIP(call)                                         \
     do {                                                      \
@@ -849,11 +854,7 @@ void ctx_release(pcs_ctx* c)
 int pcs_close(pcs_ctx* c)
 {
     if (!c) return PCS_OK;
-    if (c->oneshot) {
-        pcs_batch* b = c->oneshot;
-        c->oneshot = nullptr;
-        pcs_batch_destroy(b);
-    }
+    pcs_batch_destroy(c->oneshot.exchange(kClosed));
     ctx_release(c);
     return PCS_OK;
 }
@@ -1964,17 +1965,14 @@ int pcs_simulate(pcs_ctx* c, const pcs_proposal* props, uint32_t n, const uint32
                  uint32_t* hist_out, uint32_t* tracks_out)
 {
     if (!c) return set_error(PCS_EINVAL, "context is NULL");
-    pcs_batch* b = c->oneshot;
-    c->oneshot = nullptr;
+    pcs_batch* b = c->oneshot.exchange(nullptr);
     if (!b) PCS_TRY(pcs_batch_create(c, &b));
     int r = pcs_batch_load(b, props, n, vframes, vparticles, n_videos);
     if (r == PCS_OK) r = pcs_batch_run(b, seed, mode);
     if (r == PCS_OK) r = pcs_batch_read(b, dist_out, hist_out, tracks_out);
-    if (r == PCS_OK && b->cap_props <= kHostResults && b->cap_arena <= kOneshotKeep && !b->d_rec2) {
-        c->oneshot = b;
-    } else {
-        pcs_batch_destroy(b);
-    }
+    const bool keep = r == PCS_OK && b->cap_props <= kHostResults && b->cap_arena <= kOneshotKeep && !b->d_rec2;
+    pcs_batch* none = nullptr;
+    if (!keep || !c->oneshot.compare_exchange_strong(none, b)) pcs_batch_destroy(b);
     return r;
 }
 

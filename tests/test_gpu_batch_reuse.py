@@ -1,12 +1,15 @@
 """A batch and a context used on after a call that failed, that was empty or
 that was unusually large: what a call leaves behind must not reach the next."""
+import ctypes as C
+import threading
+
 import numpy as np
 import pytest
 
 import cases
 from part_conc_spt_abc_amd import _abi
 from part_conc_spt_abc_amd.gpu import Context
-from part_conc_spt_abc_amd.model import prior_record
+from part_conc_spt_abc_amd.model import prior_record, proposals_array
 
 pytestmark = pytest.mark.gpu
 
@@ -15,6 +18,15 @@ def population(n_pop, log10c):
     rng = np.random.default_rng(n_pop)
     theta = np.vstack([rng.uniform(0.5, 2.5, (2, n_pop)), np.full((2, n_pop), log10c), np.full((1, n_pop), 2.0)])
     return theta, np.cumsum(np.full(n_pop, 1.0 / n_pop)), np.array([0.1, 0.1, 0.0, 0.0, 0.1])
+
+
+def simulate(ctx, props, f, n, seed):
+    dist, tracks = np.empty(len(props)), np.empty(len(props), np.uint32)
+    p = lambda a: a.ctypes.data_as(C.c_void_p)  # noqa: E731
+    arr = proposals_array(props)
+    _abi.check(ctx.lib.pcs_simulate(ctx.h, C.cast(arr, C.c_void_p), len(props), p(f), p(n), len(f), seed,
+                                    _abi.PCS_MODE_BATCHED, p(dist), None, p(tracks)), "pcs_simulate")
+    return dist, tracks
 
 
 def test_propose_after_a_failed_propose(gpu_lib):
@@ -52,3 +64,33 @@ def test_propose_after_a_failed_propose(gpu_lib):
         assert all(np.array_equal(x, y) for k in (0, 1) for x, y in zip(got[k], got[k + 2]))
         c.close()
         b.close()
+
+
+def test_overlapping_one_shot_calls(gpu_lib):
+    """Calls of pcs_simulate that overlap on one context: each has a batch of
+    its own, the kept one goes to one of them only."""
+    model = cases.headline_model(n_k=60, n_de=40)
+    obs = np.zeros((60, 40), np.uint32)
+    obs[4, 7] = 3
+    loads = [cases.draw_proposals(model, k, np.random.default_rng(k), frames_choices=(30, 90), c_range=(5e7, 3e9))
+             for k in (1, 2, 7, 40, 3, 90)]
+    with Context(model, obs) as ctx:
+        want = [simulate(ctx, *w, 5) for w in loads]
+        wrong = []
+
+        def calls(i):
+            try:
+                for k in range(30):
+                    j = (i + k) % len(loads)
+                    d, t = simulate(ctx, *loads[j], 5)
+                    if not (np.array_equal(d, want[j][0]) and np.array_equal(t, want[j][1])):
+                        wrong.append((i, k))
+            except Exception as e:
+                wrong.append((i, e))
+
+        threads = [threading.Thread(target=calls, args=(i,)) for i in range(6)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        assert not wrong, wrong
