@@ -140,7 +140,11 @@ int pcs_close(pcs_ctx* ctx);
 
 /* One-shot: simulate n proposals and write log10 distances (n doubles).
  * hist_out (nullable) receives n*n_k*n_de histograms; tracks_out (nullable)
- * the number of binned tracks per proposal. Blocks until done. */
+ * the number of binned tracks per proposal. Blocks until done. The context
+ * keeps the call's buffers for the next one, until pcs_close: none of its
+ * results, and at most 32 MB of track records, 16 MB of device histogram,
+ * 16 MB of pinned staging, 8 MB of video tables and 4,096 simulations'
+ * records; a larger call's buffers are freed when it returns. */
 int pcs_simulate(pcs_ctx* ctx, const pcs_proposal* props, uint32_t n,
                  const uint32_t* video_frames, const uint32_t* video_particles, uint32_t n_videos,
                  uint64_t seed, int mode, double* dist_out, uint32_t* hist_out,

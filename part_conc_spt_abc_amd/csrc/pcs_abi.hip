@@ -279,7 +279,8 @@ int dev_alloc(T** p, size_t n)
 
 constexpr uint32_t kHostResults = 4096;
 constexpr size_t kHistKeep = 16u << 20;     // bytes
-constexpr uint64_t kOneshotKeep = 4u << 20;  // records of a kept pcs_simulate batch
+constexpr uint64_t kOneshotKeep = 4u << 20;   // records of a kept pcs_simulate batch
+constexpr size_t kOneshotVideos = 1u << 18;   // and its videos (24 bytes each on the device)
 pcs_batch* const kClosed = reinterpret_cast<pcs_batch*>(alignof(pcs_batch));  // no batch
 
 #define PCS_HIP(call)                                         \
@@ -1970,7 +1971,8 @@ int pcs_simulate(pcs_ctx* c, const pcs_proposal* props, uint32_t n, const uint32
     int r = pcs_batch_load(b, props, n, vframes, vparticles, n_videos);
     if (r == PCS_OK) r = pcs_batch_run(b, seed, mode);
     if (r == PCS_OK) r = pcs_batch_read(b, dist_out, hist_out, tracks_out);
-    const bool keep = r == PCS_OK && b->cap_props <= kHostResults && b->cap_arena <= kOneshotKeep && !b->d_rec2;
+    const bool keep = r == PCS_OK && b->cap_props <= kHostResults && b->cap_videos <= kOneshotVideos &&
+                      b->cap_arena <= kOneshotKeep && !b->d_rec2;
     pcs_batch* none = nullptr;
     if (!keep || !c->oneshot.compare_exchange_strong(none, b)) pcs_batch_destroy(b);
     return r;

@@ -94,3 +94,27 @@ def test_overlapping_one_shot_calls(gpu_lib):
         for t in threads:
             t.join()
         assert not wrong, wrong
+
+
+def free_bytes():
+    free, total = C.c_size_t(0), C.c_size_t(0)
+    assert C.CDLL("libamdhip64.so.7").hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+@pytest.mark.parametrize("particles,videos", [(0, 1 << 24), (1, 1 << 21)])
+def test_large_one_shot_leaves_no_buffers(gpu_lib, particles, videos):
+    """A call of one simulation with very many videos, empty or not: what the
+    context keeps of it stays within what pcs_abi.h states (a quarter is left
+    for the allocator)."""
+    model = cases.headline_model(n_k=60, n_de=40)
+    p, _, _ = cases.fixed_proposal(model, [1], [2])
+    with Context(model) as ctx:
+        small = np.ones(1, np.uint32)
+        simulate(ctx, [p], small, small, 1)
+        before = free_bytes()
+        p.n_videos = videos
+        simulate(ctx, [p], np.full(videos, 2, np.uint32), np.full(videos, particles, np.uint32), 1)
+        assert before - free_bytes() <= 1.25 * (64 << 20)
+        p.n_videos = 1
+        simulate(ctx, [p], small, small, 1)
