@@ -324,7 +324,8 @@ int alloc_results(pcs_batch* b, uint32_t n)
     return PCS_OK;
 }
 
-// Copies n results to the host: the stream is idle when they are already there.
+// Copies the results of n_props > 0 simulations to the host: the stream is
+// idle when they are already there.
 template <typename T>
 int fetch_results(pcs_batch* b, T* out, const T* res)
 {
@@ -598,6 +599,8 @@ bool same_tune(const pcs_tuning& a, const pcs_tuning& b) { return std::memcmp(&a
 // the next run restores them.
 int rerun_overflows(pcs_batch* b)
 {
+    b->reruns = 0;
+    if (b->n_props == 0) return PCS_OK;  // a fresh batch has no result arrays
     std::vector<int32_t> st_h;
     std::vector<uint32_t> cnt_h;
     const int32_t* st = b->d_status;
@@ -1529,7 +1532,7 @@ int pcs_batch_read_exact(pcs_batch* b, uint64_t* exact_out)
     if (!b->ran) return set_error(PCS_ESTATE, "batch has not run");
     PCS_HIP(hipSetDevice(b->ctx->device));
     PCS_HIP(hipStreamSynchronize(b->stream));
-    PCS_TRY(fetch_results(b, exact_out, b->d_exact));
+    if (b->n_props) PCS_TRY(fetch_results(b, exact_out, b->d_exact));
     PCS_HIP(hipStreamSynchronize(b->stream));
     return PCS_OK;
 }

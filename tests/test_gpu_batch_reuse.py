@@ -96,6 +96,24 @@ def test_overlapping_one_shot_calls(gpu_lib):
         assert not wrong, wrong
 
 
+def test_no_simulations(gpu_lib):
+    """A batch of no simulations runs and is read in every form, before the
+    batch has held any and after."""
+    model = cases.headline_model(n_k=60, n_de=40)
+    empty = ([], np.empty(0, np.uint32), np.empty(0, np.uint32))
+    some = cases.draw_proposals(model, 3, np.random.default_rng(1), frames_choices=(30,), c_range=(5e8, 3e9))
+    with Context(model) as ctx:
+        b = ctx.batch()
+        for load in (empty, some, empty):
+            b.load(*load)
+            for mode in range(4):
+                b.run(3, mode)
+                dist, tracks, H = b.read(hist=True)
+                assert len(dist) == len(tracks) == len(H) == len(b.read_exact()) == len(load[0])
+                assert b.overflow_reruns() == 0 and (not len(tracks) or tracks.sum() > 0)
+        b.close()
+
+
 def free_bytes():
     free, total = C.c_size_t(0), C.c_size_t(0)
     assert C.CDLL("libamdhip64.so.7").hipMemGetInfo(C.byref(free), C.byref(total)) == 0
