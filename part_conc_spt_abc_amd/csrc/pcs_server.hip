@@ -816,6 +816,9 @@ int pcs_server_create(int device, const pcs_server_config* cfg, pcs_server** out
         for (int k = 0; k < kStreams && e == hipSuccess; ++k)
             e = group_alloc(s->groups[k], s->cfg.max_inflight, s->cfg.max_inflight * s->cfg.max_videos);
     }
+    // hipMemset may return before it is done, and the groups' and the loop's
+    // streams do not wait for the null stream
+    if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
     if (e != hipSuccess) {
         const int r = hip_error(e, "pcs_server_create");
         pcs_server_destroy(s);

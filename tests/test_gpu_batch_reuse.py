@@ -1,5 +1,6 @@
 """A batch and a context used on after a call that failed, that was empty or
-that was unusually large: what a call leaves behind must not reach the next."""
+that was unusually large: what a call leaves behind must not reach the next.
+And a server's first requests, which find its buffers as it was made."""
 import ctypes as C
 import threading
 
@@ -8,7 +9,7 @@ import pytest
 
 import cases
 from part_conc_spt_abc_amd import _abi
-from part_conc_spt_abc_amd.gpu import Context
+from part_conc_spt_abc_amd.gpu import Context, Server
 from part_conc_spt_abc_amd.model import prior_record, proposals_array
 
 pytestmark = pytest.mark.gpu
@@ -136,3 +137,32 @@ def test_large_one_shot_leaves_no_buffers(gpu_lib, particles, videos):
         assert before - free_bytes() <= 1.25 * (64 << 20)
         p.n_videos = 1
         simulate(ctx, [p], small, small, 1)
+
+
+@pytest.mark.parametrize("device_loop", [False, True])
+def test_first_requests_of_a_server(gpu_lib, device_loop):
+    model = cases.headline_model(n_k=60, n_de=40)
+    obs = np.zeros((60, 40), np.uint32)
+    obs[4, 7] = 3
+    props, f, n = cases.draw_proposals(model, 9, np.random.default_rng(2), frames_choices=(30, 90), c_range=(5e7, 3e9))
+    with Context(model, obs) as ctx:
+        b = ctx.batch()
+        b.load(props, f, n)
+        b.run(5)
+        _, tracks, _ = b.read()
+        exact = b.read_exact()
+        b.close()
+    for p in props:
+        p.first_video = 0
+    for _ in range(4):
+        srv = Server(arena_bytes=1 << 24, max_inflight=16, max_videos=1, device_loop=device_loop)
+        sid = srv.add_system(model, obs)
+        for i, p in enumerate(props):
+            assert srv.submit(i, sid, p, f[i:i + 1], n[i:i + 1], 5)
+        got = {}
+        for _ in range(20000):
+            got.update((c.tag, (c.status, int(c.tracks), int(c.exact))) for c in srv.poll(64, wait_us=1000))
+            if len(got) == len(props):
+                break
+        srv.close()
+        assert [got.get(i) for i in range(len(props))] == [(0, int(t), int(x)) for t, x in zip(tracks, exact)]
