@@ -1755,11 +1755,13 @@ __device__ __forceinline__ void zero_cols(uint32_t* p)
 // 64 lanes x CPL columns, the running column sums of the cumulative histogram
 // in registers, no barrier from row to row. (The block form sweeps row after
 // row with a barrier or two each: 3 simulations of 104,000 records at H
-// 1000x1000 took 400 us, now 88.) What bounds it now are the two passes over
-// the records: LDS atomics, 8 to 12 cycles for a wave's 64. A wave's starting column sums are the
-// column histogram of the records before its first row: of the rows before the
-// workgroup's (counted by the scatter; none for part 0), plus the earlier
-// waves' histograms of their own records (counted by the scatter too).
+// 1000x1000 with 110 observed rows took 215 us, now 73; one of 4,200 records at
+// H 1000x500 with 400 observed rows 141, now 18.) What bounds it now are the two
+// passes over the records: LDS atomics, 8 to 12 cycles for a wave's 64. A wave's
+// starting column sums are the column histogram of the records before its first
+// row: of the rows before the workgroup's (counted by the scatter; none for part
+// 0), plus the earlier waves' histograms of their own records (counted by the
+// scatter too).
 //
 // The slice is read from HBM once when it holds at most KREG records a thread
 // (held in registers between the row count and the scatter); records past that
@@ -1897,9 +1899,12 @@ __device__ __forceinline__ DistOut distance_split(const DevProp& pr, const DevSy
     auto first_slot = [&](uint32_t r) -> uint32_t { return r < n_k ? rowc[row_counter(r)] : T; };  // records before row r
     const uint32_t obs_rec = uniform(first_slot(mo1));
     constexpr uint32_t kRowCost = 8u;
+    // (Rows past mo1 as a maximum less mo1: with r - mo1 in a conditional the
+    // compiler, AMD clang 22, took r >= mo1 for granted and made min(r, mo1) the
+    // constant mo1, so that one wave swept all rows of the observed table.)
     auto cost = [&](uint32_t r) -> uint32_t {
-        const uint32_t n = first_slot(r);
-        return kRowCost * (min(r, mo1) + (r > mo1 ? min(r - mo1, n - obs_rec) : 0u)) + n / 16u;
+        const uint32_t n = first_slot(r), past = max(r, mo1) - mo1;
+        return kRowCost * (min(r, mo1) + min(past, n - obs_rec)) + n / 16u;  // (n - obs_rec wraps where past is 0)
     };
     const uint64_t tot = cost(r_end);
     // first row whose cost before it reaches piece k's share
@@ -3599,17 +3604,19 @@ hipError_t launch_distance(const DistArgs& args, uint32_t n_k_max, uint32_t n_de
     DistArgs a = args;
     const uint32_t n_cu = device_cus();
     a.parts = 1u;
-    // Up to four simulations a CU the rows are split over waves; past that
-    // enough workgroups wait for each other's latency, and the block form's
-    // smaller working set (8 workgroups a CU) wins. Split against block form,
-    // H 1000x500: 300 simulations 126 against 168 us, 700: 173 against 194,
-    // 1,000: 203 both, 2,000: 316 against 270; H 1000x1000 with 73,000 records
-    // each: 61 simulations 166 against 480 us, 3: 88 against 400.
+    // Up to four simulations a CU the rows are split over waves. Split against
+    // block form with 110 observed rows, H 1000x500 and 4,500 records each: 300
+    // simulations 24 against 69 us, 700: 42 against 80, 1,024: 49 against 88; H
+    // 1000x1000: 61 simulations of 73,000 records 63 against 209 us, 3 of
+    // 104,000 73 against 215. (Nothing observed and under 50 records each, the
+    // block form is the faster one: 1 simulation 14 against 8 us, 700 19
+    // against 15.)
     if (n_de_max <= 1024u && a.n_props <= 4u * n_cu) {
         // As many workgroups share a simulation as give every CU one (more
-        // read the slice oftener than they save: 61 simulations by 4 166 us,
-        // by 8 217). Past one simulation a CU, 8 waves let two fit a CU
-        // (500 simulations: 130 us, with 16 waves 165).
+        // read the slice oftener than they save: 61 simulations of 73,000
+        // records by 4 63 us, by 8 121). Past one simulation a CU, 8 waves let
+        // two fit a CU (500 simulations of 4,500 records: 26 us, with 16 waves
+        // 33).
         if (a.scratch)
             a.parts = std::max(1u, std::min(std::min(kDistMaxParts, n_cu / a.n_props), kDistSlots / a.n_props));
         const uint32_t cpl = dist_cpl(n_de_max);
