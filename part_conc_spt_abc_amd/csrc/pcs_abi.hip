@@ -551,8 +551,9 @@ int enqueue_plain(pcs_batch* b, const std::vector<uint32_t>* subset, bool stream
         const uint32_t v0 = b->dev_planned ? P * b->J : b->props[P].first_video;
         const uint32_t lo = b->vtile[v0], hi = b->vtile[v0 + (b->dev_planned ? b->J : b->props[P].n_videos)];
         hipStream_t s = streams ? b->pstream[i % PCS_PLAIN_STREAMS] : b->stream;
-        PCS_HIP(launch_walk(walk_args(b, lo, hi), (int)t.particles_per_lane, (int)t.waves_per_group, false, 0, gauss,
-                            zref, s));
+        WalkArgs wa = walk_args(b, lo, hi);
+        wa.tile_total = nullptr;  // the plan is here: [lo, hi) is exact
+        PCS_HIP(launch_walk(wa, (int)t.particles_per_lane, (int)t.waves_per_group, false, 0, gauss, zref, s));
         PCS_HIP(launch_distance(dist_args(b, P, 1, streams ? 1 + (int)(i % PCS_PLAIN_STREAMS) : 0), c->sys.n_k, c->sys.n_de, s));
     }
     if (streams) {

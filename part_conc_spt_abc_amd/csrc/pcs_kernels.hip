@@ -3485,9 +3485,10 @@ hipError_t launch_walk(const WalkArgs& a, int ppl, int wpg, bool persistent, uin
     // 1,000 frames: 4 tiles (500 frames) 41 against 205 us, 1,000 180 against
     // 255, 1,500 260 against 298, 2,000 330 against 294, 3,500 537 against 436;
     // Gaussian at 2,000 frames 1,000 tiles 640 against 620, 2,000 1,263 against
-    // 750; at 300 frames 1,500 tiles 88 against 100, 2,000 114 against 101. (A
-    // range planned on the device is not known here, and tiles of 128 particles
-    // are not the group's.)
+    // 750; at 300 frames 1,500 tiles 88 against 100, 2,000 114 against 101.
+    // (tile_total set: a batched launch over a plan that only the device has
+    // need not know its number of tiles. Tiles of 128 particles are not the
+    // group's.)
     const uint32_t n_cu = device_cus();
     if (ppl == 1 && !a.tile_total && 4u * (uint64_t)(a.tile_hi - a.tile_lo) <= (gauss ? 15u : 27u) * n_cu) {
         const uint32_t grid = std::min(a.tile_hi - a.tile_lo, (gauss ? 1u : 2u) * n_cu);

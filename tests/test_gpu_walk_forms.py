@@ -1,0 +1,48 @@
+"""The forms of the walk against each other and the oracle, each at a number of
+tiles that reaches it: a workgroup a tile (up to 6.75 tiles a CU, 3.75 with
+Gaussian detection) and a wave a tile above, and in batches planned on the
+device."""
+import numpy as np
+import pytest
+
+import cases
+import oracle_lib as O
+from part_conc_spt_abc_amd import _abi
+from part_conc_spt_abc_amd.gpu import Context
+from part_conc_spt_abc_amd.model import prior_record
+
+pytestmark = pytest.mark.gpu
+
+CLASSES = {
+    "slab": {},
+    "slab, walls": dict(z_boundary=_abi.PCS_Z_REFLECT),
+    "gauss": dict(detect_model=_abi.PCS_DETECT_GAUSS_Z, detect_sigma=1.5),
+    "gauss, walls": dict(detect_model=_abi.PCS_DETECT_GAUSS_Z, detect_sigma=1.5, z_boundary=_abi.PCS_Z_REFLECT),
+}
+
+
+@pytest.mark.parametrize("ppl", [1, 2])
+@pytest.mark.parametrize("cls", list(CLASSES))
+def test_plain_launches_of_proposed_trials(gpu_lib, cls, ppl):
+    """Proposed trials in the batched form (the device's plan) and one by one
+    (the host has fetched it), with slices that fit and slices that overflow."""
+    model = cases.headline_model(n_k=140, n_de=64, Lz=15.0, **CLASSES[cls])
+    rng = np.random.default_rng(2)
+    theta = np.vstack([rng.uniform(0.5, 2.5, (2, 20)), rng.uniform(7.5, 9.0, (2, 20)), np.full((1, 20), 8.0)])
+    pr = prior_record(model, (0.1, 5.0), (6.5, 9.5), (0.5, 14.0))
+    frames = rng.integers(2, 140, (37, 3)).astype(np.uint32)
+    with Context(model) as ctx:
+        ctx.set_tuning(particles_per_lane=ppl)
+        got = []
+        for factor in (0.5, 1e-4):
+            ctx.set_record_capacity_factor(factor)
+            b = ctx.batch()
+            b.propose(pr, theta, np.cumsum(np.full(20, 0.05)), np.full(5, 0.1), 37, frames, seed=5)
+            for mode in (_abi.PCS_MODE_BATCHED, _abi.PCS_MODE_PLAIN, _abi.PCS_MODE_PLAIN_STREAMS):
+                b.run(9, mode)
+                _, tracks, H = b.read(hist=True)
+                got.append((tracks, H, b.read_exact()))
+                assert (b.overflow_reruns() > 0) == (factor < 0.1)
+            b.close()
+    assert int(got[0][0].sum()) > 1000
+    assert all(np.array_equal(x, y) for g in got[1:] for x, y in zip(g, got[0]))
