@@ -2222,6 +2222,14 @@ __device__ __forceinline__ DistOut split_any(const DevProp& pr, const DevSys& sy
     return distance_split<CPL, NW, KREG>(pr, sy, count, L, part, parts);
 }
 
+// Where the passes over the records and the sweep are this short, one workgroup
+// has done both before several have shared them out and their sums are added up.
+// One against 16 workgroups, one simulation at H 1000x500: nothing observed and
+// 49 records 10.8 against 14.6 us, 110 observed rows and 456 records 12.9
+// against 13.8, with 4,000 records 14.8 both; H 1000x1000, 110 rows and 2,100
+// records 19.7 against 18.8, 255 rows 27.8 against 19.4.
+constexpr uint32_t kSplitAloneRecords = 2048, kSplitAloneRows = 128;
+
 // `a.parts` workgroups of NW waves per simulation (neighbouring blocks), whose
 // sums the last to finish adds up. Dynamic LDS as laid out by SplitLds, sized
 // to the models of the launch.
@@ -2240,19 +2248,26 @@ __global__ __launch_bounds__(NW * kWave) void distance_split_kernel(DistArgs a)
     const uint32_t job = blockIdx.x / a.parts, part = blockIdx.x % a.parts;
     const uint32_t P = a.prop_lo + job;
     const DevProp& pr = a.props[P];
-    DistOut o = split_any<CPL, NW, 8>(pr, a.sys[pr.sys_id], a.rec_count[P], L, part, a.parts);
+    const DevSys& sy = a.sys[pr.sys_id];
+    const uint32_t count = a.rec_count[P];
+    uint32_t parts = a.parts;
+    if (parts > 1u && count <= kSplitAloneRecords && sy.maxrow_obs < kSplitAloneRows) {
+        if (part != 0u) return;
+        parts = 1u;
+    }
+    DistOut o = split_any<CPL, NW, 8>(pr, sy, count, L, part, parts);
     if (threadIdx.x != 0) return;
-    if (a.parts > 1u) {
+    if (parts > 1u) {
         if (o.status == PCS_OK) {
             uint64_t* slot = a.scratch->sum + 2u * (uint64_t)blockIdx.x;
             st_agent64(slot, o.lo);
             st_agent64(slot + 1, o.hi);
             const uint32_t t = __hip_atomic_fetch_add(&a.scratch->ticket[job], 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-            if (t + 1u != a.parts) return;
+            if (t + 1u != parts) return;
             st_agent32(&a.scratch->ticket[job], 0u);  // as the next launch expects it
             o.lo = o.hi = 0ull;
-            for (uint32_t q = 0; q < a.parts; ++q) {
-                const uint64_t* s = a.scratch->sum + 2u * ((uint64_t)job * a.parts + q);
+            for (uint32_t q = 0; q < parts; ++q) {
+                const uint64_t* s = a.scratch->sum + 2u * ((uint64_t)job * parts + q);
                 add128(o.lo, o.hi, ld_agent64(s), ld_agent64(s + 1));
             }
         } else if (part != 0u) {
@@ -3610,8 +3625,10 @@ hipError_t launch_distance(const DistArgs& args, uint32_t n_k_max, uint32_t n_de
     // simulations 24 against 69 us, 700: 42 against 80, 1,024: 49 against 88; H
     // 1000x1000: 61 simulations of 73,000 records 63 against 209 us, 3 of
     // 104,000 73 against 215. (Nothing observed and under 50 records each, the
-    // block form is the faster one: 1 simulation 14 against 8 us, 700 19
-    // against 15.)
+    // block form is the faster one: 1 simulation 10 against 8 us, 700 19
+    // against 15.) Past it the block form is kept: 2,000 simulations of 4,500
+    // records 135 us, split 90; with nothing observed and 44 records each 34,
+    // split 49, and 8,000 of them 102 and 158.
     if (n_de_max <= 1024u && a.n_props <= 4u * n_cu) {
         // As many workgroups share a simulation as give every CU one (more
         // read the slice oftener than they save: 61 simulations of 73,000
