@@ -3248,7 +3248,8 @@ __global__ __launch_bounds__(kPmcBlock) void pmc_sums_kernel(const double* __res
 // kept off it: in round i waves 1..3 load tile i into LDS and store tile
 // i - 2's sums, while lane 0 adds through tile i - 1 in place, 16 weights read
 // ahead of the 16 being added. Bound by the additions' latency. (Each weight
-// broadcast by readlane between the additions, 100,000 members took 4.4 ms.)
+// broadcast by readlane between the additions, 100,000 members took 4.4 ms, now
+// 1.0.)
 constexpr uint32_t kCumTile = 2048;
 __global__ __launch_bounds__(256) void cumsum_kernel(const double* w, uint32_t n, double* cum)
 {
@@ -3274,23 +3275,28 @@ __global__ __launch_bounds__(256) void cumsum_kernel(const double* w, uint32_t n
             f64x2 a[8], b[8];
 #pragma unroll
             for (int q = 0; q < 8; ++q) a[q] = p[q];
-            for (uint32_t j = 0; j < kCumTile / 2u; j += 8u) {
-                const uint32_t nx = min(j + 8u, kCumTile / 2u - 8u);
+            auto add = [&](uint32_t end) {
+                for (uint32_t j = 0; j < end; j += 8u) {
+                    const uint32_t nx = min(j + 8u, end - 8u);
 #pragma unroll
-                for (int q = 0; q < 8; ++q) b[q] = p[nx + q];
+                    for (int q = 0; q < 8; ++q) b[q] = p[nx + q];
 #pragma unroll
-                for (int q = 0; q < 8; ++q) {
-                    acc += a[q].x;
-                    a[q].x = acc;
-                    acc += a[q].y;
-                    a[q].y = acc;
+                    for (int q = 0; q < 8; ++q) {
+                        acc += a[q].x;
+                        a[q].x = acc;
+                        acc += a[q].y;
+                        a[q].y = acc;
+                    }
+#pragma unroll
+                    for (int q = 0; q < 8; ++q) {
+                        p[j + q] = a[q];
+                        a[q] = b[q];
+                    }
                 }
-#pragma unroll
-                for (int q = 0; q < 8; ++q) {
-                    p[j + q] = a[q];
-                    a[q] = b[q];
-                }
-            }
+            };
+            // whole tiles in a loop of known length; the last one up to n
+            if (it < nt) add(kCumTile / 2u);
+            else add((n - (nt - 1u) * kCumTile + 15u) / 16u * 8u);
         }
         __syncthreads();
     }
