@@ -280,7 +280,11 @@ int pcs_get_tuning(pcs_ctx* ctx, pcs_tuning* t);
  * per CU {2,4,6,8,12,16} (those the hardware can co-schedule) - and keeps
  * the fastest in the context. best/ms (nullable) receive the winner and its
  * walk time (the faster of 2 runs; one untimed run warms each kernel first).
- * Results never depend on the shape. */
+ * Proposals of so few tiles that each is walked by a workgroup of its own (up
+ * to 6.75 tiles of 64 particles per CU, 3.75 with Gaussian detection) say
+ * nothing about the shape: with one particle per lane the fastest, waves per
+ * group and groups per CU then stay as they are. Results never depend on the
+ * shape. */
 int pcs_autotune(pcs_ctx* ctx, const pcs_proposal* props, uint32_t n, const uint32_t* video_frames,
                  const uint32_t* video_particles, uint32_t n_videos, pcs_tuning* best, float* ms);
 

@@ -1638,6 +1638,7 @@ int pcs_autotune(pcs_ctx* c, const pcs_proposal* props, uint32_t n, const uint32
     pcs_tuning best = saved;
     float best_ms = -1.0f;
     int r = pcs_batch_load(b, props, n, vframes, vparticles, n_videos);
+    const bool gauss = c->sys.detect_model == PCS_DETECT_GAUSS_Z;
     for (uint32_t ppl : {1u, 2u}) {
         bool warm = false;  // one untimed run per kernel (particles per lane)
         for (uint32_t wpg : {2u, 4u}) {
@@ -1646,10 +1647,11 @@ int pcs_autotune(pcs_ctx* c, const pcs_proposal* props, uint32_t n, const uint32
                 if (wpg * gpc > 32u) continue;  // more waves than a CU holds (8 per SIMD)
                 pcs_tuning t{ppl, wpg, gpc, saved.stage_records};
                 c->tune = t;
-                if (!warm) {
-                    r = pcs_batch_run(b, 0x5eedull, PCS_MODE_BATCHED_DIRECT);
-                    warm = true;
-                }
+                if (!warm) r = pcs_batch_run(b, 0x5eedull, PCS_MODE_BATCHED_DIRECT);
+                // (n_tiles: of this many particles a lane, from the run on)
+                const bool groups = walk_by_groups(b->n_tiles, (int)ppl, gauss);
+                if (groups && warm) continue;  // one kernel for all of these shapes
+                warm = true;
                 float t_ms = -1.0f;  // the faster of two timed runs
                 for (int k = 1; k <= 2 && r == PCS_OK; ++k) {
                     r = pcs_batch_run(b, 0x5eedull + (uint64_t)k, PCS_MODE_BATCHED_DIRECT);
@@ -1661,6 +1663,10 @@ int pcs_autotune(pcs_ctx* c, const pcs_proposal* props, uint32_t n, const uint32
                 if (best_ms < 0.0f || t_ms < best_ms) {
                     best_ms = t_ms;
                     best = t;
+                    if (groups) {  // a choice of particles a lane, not of a shape
+                        best.waves_per_group = saved.waves_per_group;
+                        best.groups_per_cu = saved.groups_per_cu;
+                    }
                 }
             }
         }

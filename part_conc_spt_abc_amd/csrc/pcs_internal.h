@@ -285,6 +285,9 @@ struct ProposeArgs {
 
 // Launchers (pcs_kernels.hip). waves_per_group in {1,2,4}; ppl in {1,2}.
 hipError_t launch_reset(uint32_t* rec_count, uint32_t n, uint32_t* tile_counter, hipStream_t s);
+// walk_by_groups: that many tiles are walked by a workgroup each, whatever
+// waves_per_group and grid_groups say.
+bool walk_by_groups(uint32_t tiles, int ppl, bool gauss);
 hipError_t launch_walk(const WalkArgs& a, int ppl, int waves_per_group, bool persistent,
                        uint32_t grid_groups, bool gauss, bool zreflect, hipStream_t s);
 hipError_t launch_distance(const DistArgs& a, uint32_t n_k_max, uint32_t n_de_max, hipStream_t s);

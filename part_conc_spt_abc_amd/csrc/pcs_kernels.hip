@@ -3497,21 +3497,26 @@ static hipError_t launch_group_t(const WalkArgs& a, uint32_t grid, hipStream_t s
     return hipGetLastError();
 }
 
+// Few tiles: a workgroup each, as long as that beats a wave each: up to 6.75
+// tiles a CU, 3.75 with Gaussian detection. Group against wave at 1,000 frames:
+// 4 tiles (500 frames) 41 against 205 us, 1,000 180 against 255, 1,500 260
+// against 298, 2,000 330 against 294, 3,500 537 against 436; Gaussian at 2,000
+// frames 1,000 tiles 640 against 620, 2,000 1,263 against 750; at 300 frames
+// 1,500 tiles 88 against 100, 2,000 114 against 101. (Tiles of 128 particles are
+// not the group's.)
+bool walk_by_groups(uint32_t tiles, int ppl, bool gauss)
+{
+    return ppl == 1 && 4u * (uint64_t)tiles <= (gauss ? 15u : 27u) * device_cus();
+}
+
 hipError_t launch_walk(const WalkArgs& a, int ppl, int wpg, bool persistent, uint32_t grid_groups,
                        bool gauss, bool zref, hipStream_t s)
 {
     if (a.tile_hi <= a.tile_lo) return hipSuccess;
-    // Few tiles: a workgroup each, as long as that beats a wave each: up to
-    // 6.75 tiles a CU, 3.75 with Gaussian detection. Group against wave at
-    // 1,000 frames: 4 tiles (500 frames) 41 against 205 us, 1,000 180 against
-    // 255, 1,500 260 against 298, 2,000 330 against 294, 3,500 537 against 436;
-    // Gaussian at 2,000 frames 1,000 tiles 640 against 620, 2,000 1,263 against
-    // 750; at 300 frames 1,500 tiles 88 against 100, 2,000 114 against 101.
-    // (tile_total set: a batched launch over a plan that only the device has
-    // need not know its number of tiles. Tiles of 128 particles are not the
-    // group's.)
     const uint32_t n_cu = device_cus();
-    if (ppl == 1 && !a.tile_total && 4u * (uint64_t)(a.tile_hi - a.tile_lo) <= (gauss ? 15u : 27u) * n_cu) {
+    // (tile_total set: a batched launch over a plan that only the device has
+    // need not know its number of tiles.)
+    if (!a.tile_total && walk_by_groups(a.tile_hi - a.tile_lo, ppl, gauss)) {
         const uint32_t grid = std::min(a.tile_hi - a.tile_lo, (gauss ? 1u : 2u) * n_cu);
         if (gauss) return zref ? launch_group_t<true, true>(a, grid, s) : launch_group_t<true, false>(a, grid, s);
         return zref ? launch_group_t<false, true>(a, grid, s) : launch_group_t<false, false>(a, grid, s);

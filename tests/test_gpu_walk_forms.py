@@ -46,3 +46,16 @@ def test_plain_launches_of_proposed_trials(gpu_lib, cls, ppl):
             b.close()
     assert int(got[0][0].sum()) > 1000
     assert all(np.array_equal(x, y) for g in got[1:] for x, y in zip(g, got[0]))
+
+
+@pytest.mark.parametrize("cls", ["slab", "gauss, walls"])
+def test_autotune_on_few_tiles(gpu_lib, cls):
+    """Few tiles are walked by a workgroup each, whatever the shape: tuning on
+    them leaves the shape alone (one wave a group is none of the candidates)."""
+    model = cases.headline_model(n_k=140, n_de=64, Lz=15.0, **CLASSES[cls])
+    p, f, n = cases.fixed_proposal(model, [1000], [500])
+    with Context(model) as ctx:
+        ctx.set_tuning(particles_per_lane=2, waves_per_group=1, groups_per_cu=7, stage_records=128)
+        best, ms = ctx.autotune([p], f, n)
+        assert best == ctx.get_tuning() == dict(particles_per_lane=1, waves_per_group=1, groups_per_cu=7, stage_records=128)
+        assert ms > 0.0
