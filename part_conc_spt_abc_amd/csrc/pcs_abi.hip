@@ -359,7 +359,9 @@ int check_tuning(const pcs_tuning& t)
 }
 
 // Tiles beyond which the order of the videos no longer matters: 16 rounds of
-// the GPU's 8,192 wave slots. Up to two tiles a CU all of them start at once.
+// 256 CUs' 8,192 wave slots. Up to two tiles a CU the videos stay as they are:
+// all tiles start at once (Gaussian detection: one a CU at once, so above one a
+// CU in two rounds).
 constexpr uint32_t kOrderTiles = 16u * 8192u;
 
 // Tiles of 64*ppl particles per video, prefix-summed. Videos of different
@@ -1158,8 +1160,10 @@ int pcs_batch_overflow_reruns(pcs_batch* b, uint32_t* n)
 }
 
 // Dense histograms, formed from the records in chunks of proposals. They come
-// back through pinned staging, copied out while the next piece is on its way:
-// copies of megabytes into pageable memory took 0.6 to 4 ms for 2 MB.
+// back through pinned staging in pieces of up to 8 MB (kHistKeep / 8 words), each
+// copied out while the next is on its way; up to 8 MB it is one piece, copied
+// out once it is here. Copies of megabytes into pageable memory took 0.6 to 4 ms
+// for 2 MB.
 static int read_hist(pcs_batch* b, uint32_t* hist_out)
 {
     pcs_ctx* c = b->ctx;
